@@ -223,6 +223,10 @@ int kx_gemm_splitk_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, 
                         int64_t ldr, const float* gate, int64_t gate_div, int64_t gate_stride, void* workspace,
                         int64_t workspace_bytes, int splits, kx_stream_t stream);
 
+/* *splits = the number of K slices (1, 2, 4, 8 or 16) in which an (m, n, k) product is fastest: 1 for
+ * kx_gemm_bf16, more for kx_gemm_splitk_bf16 with a workspace of splits * m * n * 4 bytes. A pure
+ * function of the sizes; no GPU call. */
+int kx_gemm_splits(int64_t m, int64_t n, int64_t k, int* splits);
 /* Size of the static device array kx_gemm_splitk_noalloc_bf16 keeps its partial products in. */
 #define KX_SPLITK_SCRATCH_BYTES (16ll << 20)
 

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from functools import lru_cache
 from pathlib import Path
 
 import torch
@@ -81,6 +82,7 @@ SIGNATURES: dict[str, list] = {
     "kx_gemm_splitk_bf16": [
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _I64, _P, _I64, _I, _P,
     ],
+    "kx_gemm_splits": [_I64, _I64, _I64, _P],
     "kx_gemm_splitk_noalloc_bf16": [
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _I64, _I, _P,
     ],
@@ -564,20 +566,21 @@ def tail_split(m: int, n: int, k: int) -> tuple[int, int] | None:
     return (rows, splits) if splits > 1 else None
 
 
+@lru_cache(maxsize=4096)
 def splitk_splits(m: int, n: int, k: int) -> int:
-    """K slices for a product whose output tiles (64 x 128) leave most of the 256 CUs idle:
-    the most slices (up to 16) that keep at most 512 workgroups, a slice of at least 256 and a
-    whole number of 64-wide stages per slice; 1 means no split."""
-    if m > 512 or n <= 64 or n % 4 or k < 1024:
+    """K slices of a product (1: none): the count the library's cost rule finds fastest with the
+    reduction of the partial products included (``kx_gemm_splits``). A few-column product of many
+    rows keeps one slice, so that its rows sum in the same order however many of them a call has."""
+    if n <= 64 or n % 4 or k < 1024 or k % 64 or (m > 512 and n < 1024):
         return 1
     tiles = -(-m // 64) * -(-n // 128)
-    if tiles >= 128:
-        return 1
-    best = 1
-    for splits in (2, 4, 8, 16):
-        if tiles * splits <= 512 and k % (64 * splits) == 0 and k // splits >= 256:
-            best = splits
-    return best
+    if tiles <= 32 and k >= 8192:
+        # few 64 x 128 tiles over a long K: the most slices (up to 16) of at least 256
+        return max(s for s in (1, 2, 4, 8, 16) if k % (64 * s) == 0 and (s == 1 or k // s >= 256))
+    out = ctypes.c_int(1)
+    if load().kx_gemm_splits(m, n, k, ctypes.addressof(out)) != KX_OK:
+        raise KernelError(f"kx_gemm_splits: bad shape ({m}, {n}, {k})")
+    return out.value
 
 
 def launch_qgemm(a, words, scales, biases, out, *, n, k, group_size, bits, bias=None,

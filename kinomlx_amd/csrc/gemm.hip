@@ -1,10 +1,12 @@
-// Dense bf16 and affine int4/int8 weight-quantized linear layers on gfx950 MFMA.
+// Linear layers on gfx950 MFMA: the entry points, the affine int4 / int8 and mxfp8 weight-quantized
+// products, the few-column (gate logit) products, and the register-staged fallback. Dense products with
+// K % 64 == 0 run in gemm_dense.hip.
 //
 // c[m, n] = epilogue(sum_k a[m, k] * w[n, k]) — both operands K-contiguous (the reference's
-// (out, in) weight layout), fp32 accumulation in v_mfma_f32_32x32x16_bf16 (or _f16: the dense
-// kernels take bf16 or fp16 operands, template H), one rounding to the 16-bit type.
+// (out, in) weight layout), fp32 accumulation, one rounding to the 16-bit type (bf16, or fp16 for
+// dense operands, template H).
 //
-// Tiling: a BM x BN output tile per workgroup of WM x WN waves; each wave owns a
+// The register-staged kernel (v_mfma_f32_32x32x16): a BM x BN output tile per workgroup of WM x WN waves; each wave owns a
 // (BM/WM) x (BN/WN) sub-tile as a grid of 32x32 MFMA blocks. K advances in stages of 64: the
 // next stage's global loads are issued into registers before the current stage's MFMAs and
 // written to the other half of a double-buffered LDS tile afterwards, so one barrier per stage
@@ -26,40 +28,13 @@
 #include <mutex>
 #include <type_traits>
 
-#include "common.h"
+#include "gemm.h"
 
 namespace kx {
 namespace {
 
 constexpr int BK = 64;        // K per stage
 constexpr int ROWB = BK * 2;  // bytes per LDS tile row
-
-struct Epilogue {
-  const uint16_t* bias;
-  const void* resid;  // bf16, or fp32 with KX_EPI_RESID_F32
-  int64_t ldr;
-  const float* gate;
-  int64_t gate_div;
-  int64_t gate_stride;
-  int flags;
-  // KX_EPI_QK_NORM_ROPE: columns [0, q_end) are query heads and [q_end, k_end) key heads of 128;
-  // each row's head is RMS-normalized (weights nq / nk, fp32 or bf16, plus w_off; eps), then
-  // rotated in adjacent pairs by the row's cos / sin table row:
-  // tables + (m / t_rows) * t_bs + (m % t_rows) * t_ld + head * t_hs + d.
-  const void* nq;
-  const void* nk;
-  int n_bf16;
-  float n_eps, n_off;
-  int64_t q_end, k_end;
-  // set by the launcher, not part of the C ABI: visit the tile rows last to first (see
-  // rows_last_first)
-  int rows_desc;
-  const float* cosp;
-  const float* sinp;
-  int64_t t_ld, t_hs, t_rows, t_bs;
-  uint32_t t_magic;  // m / t_rows = (umulhi(m, t_magic) + m) >> t_shift for m < 2^31
-  int t_shift;
-};
 
 struct QuantW {
   const uint32_t* words;  // (n, k * bits / 32)
@@ -88,16 +63,6 @@ __device__ __forceinline__ uint2 mx8_quad(uint32_t w, float scale) {
 }
 
 __device__ __forceinline__ int lds_off(int r, int c) { return r * ROWB + ((c ^ (r & 7)) << 4); }
-
-__device__ __forceinline__ float apply_act(float v, int act) {
-  switch (act) {
-    case 1: return fast_gelu_tanh(v);
-    case 2: return fast_silu(v);
-    case 3: return fast_sigmoid2(v);
-    case 4: return fast_sigmoid(v);
-    default: return v;
-  }
-}
 
 template <int BITS>
 __device__ __forceinline__ uint4 dequant8(const uint32_t* wd, float s, float b) {
@@ -457,169 +422,28 @@ __global__ __launch_bounds__(256) void dequant_mx8_t_kernel(const uint32_t* __re
   }
 }
 
-// Tile of workgroup `bid` for the direct-to-LDS kernel, as (tile row, tile column). The 256
-// workgroups of a round run at once, 32 per XCD, and the XCDs' L2s are separate. When the tile
-// columns divide a round (8, 16, 32 or 64 of them) and the rows fill whole rounds, each round
-// covers R = 256 / tiles_n whole tile rows, and each XCD an a x b block of them with the fewest
-// operand panels (a + b = 12 for 32 tiles): every activation panel is then read in one round
-// only, so a product whose operands exceed the last-level cache re-reads them from HBM once per
-// round rather than once per round and XCD pair (the 9216 x 4096 x 16384 down projection: mean
-// L1 -> L2 request latency 688 -> 505 cycles, 2.5 % faster). Otherwise: XCD-contiguous tiles,
-// grouped by 8 tile rows.
-__device__ __forceinline__ int2 lds_tile_of(int bid, int tiles_m, int tiles_n) {
-  const int rows = 256 / tiles_n;
-  if ((tiles_n == 8 || tiles_n == 16 || tiles_n == 32 || tiles_n == 64) && tiles_m % rows == 0) {
-    // XCD x: block (x % ra, x / ra) of an ra x cb grid over the round, ra * cb = 8
-    const int ra = tiles_n >= 32 ? 1 : tiles_n == 16 ? 2 : 8, cb = 8 / ra;
-    const int a = rows / ra, b = tiles_n / cb;  // block rows x columns, a * b = 32
-    const int x = bid % 8, i = bid / 8, r = i / 32, j = i % 32;
-    return make_int2(r * rows + (x % ra) * a + j % a, (x / ra) * b + j / a);
-  }
-  const int t = xcd_remap(bid, tiles_m * tiles_n);
-  constexpr int GM = 8;
-  const int group_width = GM * tiles_n;
-  const int first_m = (t / group_width) * GM;
-  const int gsz = min(tiles_m - first_m, GM);
-  return make_int2(first_m + (t % group_width) % gsz, (t % group_width) / gsz);
-}
-
-// ---- direct-to-LDS pipelined kernel (dense: K % 64 == 0; quantized: K % 128 == 0) ------------
+// ---- quantized direct-to-LDS kernel (K % 128 == 0) -----------------------------------------------
 //
-// Operand tiles go from global memory straight into LDS with global_load_lds_dwordx4 (no VGPR
-// staging): one wave instruction fills 64 lanes x 16 B = DRPI rows of DBK bf16, from a scalar tile
-// base plus a loop-invariant 32-bit lane offset. Dense products use stages of DBK = 64 along K: a row's 128 bytes of a stage are one full cache line, so each row makes one
-// 128-byte L1 -> L2 request. The per-CU operand stream is bounded by the requests it keeps in
-// flight times their latency, so 128-byte requests carry twice the bytes of the 64-byte ones
-// that 32-wide stages make. The 256 x 256 and 192 x 256 tiles keep two stages in LDS: stage kt+2
-// goes into stage kt's buffer, half of its DMA instructions right after the barrier of stage
-// kt's last k16 step and half during stage kt+1's first step. The small tiles (whose few MFMAs
-// per stage cannot hide a one-stage prefetch) keep a ring of four, and so do the quantized
-// products with 32-wide stages: their DMA for stage kt+3 goes out between the MFMAs of stage kt. Every k16 step is one scheduling region: wait for this step's
-// fragments (read one step earlier), issue the fragment reads of the next step, then the step's
-// MFMAs, so LDS latency hides under a full step of MFMAs and never more than MB + NB reads are
-// outstanding (lgkmcnt counts to 15). The last step of a stage holds the stage's only workgroup
-// barrier. The 16-byte slots of a row are XOR-swizzled so that both the DMA writes and the
-// 32-row fragment reads are bank-conflict free.
+// Operand tiles go from global memory straight into LDS (no VGPR staging): one wave instruction fills
+// 64 lanes x 16 B = DRPI rows of DBK bf16, from a scalar tile base plus a loop-invariant 32-bit lane
+// offset. A ring of four stages of 32 along K; the DMA for stage kt+3 goes out between the MFMAs of
+// stage kt. Every k16 step is one scheduling region: wait for this step's fragments (read one step
+// earlier), issue the fragment reads of the next step, then the step's MFMAs, so LDS latency hides
+// under a full step of MFMAs and never more than MB + NB reads are outstanding (lgkmcnt counts to
+// 15). The last step of a stage holds the stage's only workgroup barrier. The 16-byte slots of a
+// row are XOR-swizzled so that both the DMA writes and the 32-row fragment reads are bank-conflict
+// free.
 //
 // Epilogue: each wave stages half of its fp32 tile in LDS at a time and writes it back in rows,
 // 4 columns per lane, so bias / gate / residual loads and the stores are contiguous runs. Full,
 // aligned tiles take a compile-time specialisation per residual mode (GMODE 0: none, 1: bf16
 // residual, 2: fp32 residual) and output type; edge tiles take the generic masked path.
 
-// K per LDS stage of a dense product: a row's 128 bytes per stage are one full cache line, so
-// every DMA lane group of a row makes one 128-byte request (32-wide stages made two 64-byte
-// requests per line, twice the L1 -> L2 requests for the same bytes)
-constexpr int DENSE_BK = 64;
 // 8-bit packed weight rows (32 bytes per stage): chunk swizzle of row r
 __device__ __forceinline__ int qswz(int r) { return (r >> 3) & 1; }
-#define KX_LDS(p) ((__attribute__((address_space(3))) void*)(p))
-// Raw buffer resource over `base` (stride 0, 4 GiB range; dword 3 as for every gfx9 raw buffer)
-// and a 16-byte-per-lane buffer load into LDS (M0 + lane * 16) from base + voff + soff: the
-// offsets are one loop-invariant 32-bit lane offset and a scalar K offset, so a DMA issue needs
-// no 64-bit address arithmetic (3 % on the block GEMMs against global_load_lds with per-issue
-// 64-bit VALU adds). The host compilation pass has no buffer builtins; kernels only run on the
-// device.
-#if defined(__HIP_DEVICE_COMPILE__)
-using rsrc_t = __amdgpu_buffer_rsrc_t;
-__device__ __forceinline__ rsrc_t raw_rsrc(const void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, -1, 0x00020000);
-}
-__device__ __forceinline__ void buffer_lds16(rsrc_t r, void* lds, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, KX_LDS(lds), 16, voff, soff, 0, 0);
-}
-#else
-struct rsrc_t {};
-__device__ inline rsrc_t raw_rsrc(const void*) { return {}; }
-__device__ inline void buffer_lds16(rsrc_t, void*, uint32_t, uint32_t) {}
-#endif
-// A workgroup barrier that the compiler may not move memory accesses across.
-#define KX_BARRIER() asm volatile("s_barrier" ::: "memory")
-
-// gfx9 s_waitcnt immediate that waits for vmcnt <= N only.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-__device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-// gfx9 s_waitcnt immediate that waits for lgkmcnt <= N only (LDS reads complete in order).
-template <int N>
-__device__ __forceinline__ void wait_lgkmcnt() {
-  static_assert(N >= 0 && N < 16, "lgkmcnt");
-  __builtin_amdgcn_s_waitcnt(0xC07F | (N << 8));
-}
-
-// bias + activation + gated residual on 4 consecutive columns n..n+3 of row m, then the store.
-template <bool H>
-__device__ __forceinline__ void epilogue_store4(float v[4], int m, int n, int N, const Epilogue& epi,
-                                                void* __restrict__ C, int64_t ldc, bool vec_ok) {
-  const int act = (epi.flags >> 4) & 15;
-  const bool gated = epi.flags & KX_EPI_GATED_RESIDUAL;
-  const bool resid_f32 = epi.flags & KX_EPI_RESID_F32;
-  const bool out_f32 = epi.flags & KX_EPI_OUT_F32;
-  const int64_t ro = (int64_t)m * epi.ldr + n;
-  const int64_t co = (int64_t)m * ldc + n;
-  if (vec_ok && n + 3 < N) {
-    if (epi.flags & KX_EPI_BIAS) {
-      const uint2 bb = *reinterpret_cast<const uint2*>(epi.bias + n);
-      v[0] += e_lo<H>(bb.x); v[1] += e_hi<H>(bb.x); v[2] += e_lo<H>(bb.y); v[3] += e_hi<H>(bb.y);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = apply_act(v[e], act);
-    if (gated) {
-      const float4 gv = *reinterpret_cast<const float4*>(epi.gate + (m / epi.gate_div) * epi.gate_stride + n);
-      float rv[4];
-      if (resid_f32) {
-        const float4 rr = *reinterpret_cast<const float4*>(static_cast<const float*>(epi.resid) + ro);
-        rv[0] = rr.x; rv[1] = rr.y; rv[2] = rr.z; rv[3] = rr.w;
-      } else {
-        const uint2 rr = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(epi.resid) + ro);
-        rv[0] = e_lo<H>(rr.x); rv[1] = e_hi<H>(rr.x); rv[2] = e_lo<H>(rr.y); rv[3] = e_hi<H>(rr.y);
-      }
-      v[0] = rv[0] + gv.x * v[0];
-      v[1] = rv[1] + gv.y * v[1];
-      v[2] = rv[2] + gv.z * v[2];
-      v[3] = rv[3] + gv.w * v[3];
-    }
-    if (out_f32) {
-      *reinterpret_cast<float4*>(static_cast<float*>(C) + co) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
-      uint2 o;
-      o.x = e_pack2<H>(v[0], v[1]);
-      o.y = e_pack2<H>(v[2], v[3]);
-      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(C) + co) = o;
-    }
-    return;
-  }
-  for (int e = 0; e < 4 && n + e < N; ++e) {
-    float x = v[e];
-    if (epi.flags & KX_EPI_BIAS) x += e2f<H>(epi.bias[n + e]);
-    x = apply_act(x, act);
-    if (gated) {
-      const float rv = resid_f32 ? static_cast<const float*>(epi.resid)[ro + e]
-                                 : e2f<H>(static_cast<const uint16_t*>(epi.resid)[ro + e]);
-      x = rv + epi.gate[(m / epi.gate_div) * epi.gate_stride + n + e] * x;
-    }
-    if (out_f32)
-      static_cast<float*>(C)[co + e] = x;
-    else
-      static_cast<uint16_t*>(C)[co + e] = f2e<H>(x);
-  }
-}
-
-// The activation as a compile-time choice (ACT = the epilogue's activation code; -1: chosen at
-// run time per value).
-template <int ACT>
-__device__ __forceinline__ float act_c(float v, int act) {
-  if constexpr (ACT == 1) return fast_gelu_tanh(v);
-  else if constexpr (ACT == 2) return fast_silu(v);
-  else if constexpr (ACT == 0) return v;
-  else return apply_act(v, act);
-}
-
 // One full-tile epilogue row piece: bias + activation (+ gated residual), then the store of 4
 // consecutive columns. Values by value so that nothing of the caller's frame is addressed.
-template <bool H, int GMODE, bool OUTF32, int ACT, typename ResidT>
+template <int GMODE, bool OUTF32, int ACT, typename ResidT>
 __device__ __forceinline__ void epi_row4(float4 a4, ResidT res, float b0, float b1, float b2, float b3,
                                          int act, float4 gv, char* dst) {
   float v[4] = {a4.x + b0, a4.y + b1, a4.z + b2, a4.w + b3};
@@ -632,7 +456,7 @@ __device__ __forceinline__ void epi_row4(float4 a4, ResidT res, float b0, float 
     if constexpr (GMODE == 2) {
       rv[0] = res.x; rv[1] = res.y; rv[2] = res.z; rv[3] = res.w;
     } else {
-      rv[0] = e_lo<H>(res.x); rv[1] = e_hi<H>(res.x); rv[2] = e_lo<H>(res.y); rv[3] = e_hi<H>(res.y);
+      rv[0] = lo_f(res.x); rv[1] = hi_f(res.x); rv[2] = lo_f(res.y); rv[3] = hi_f(res.y);
     }
     v[0] = rv[0] + gv.x * v[0];
     v[1] = rv[1] + gv.y * v[1];
@@ -643,81 +467,63 @@ __device__ __forceinline__ void epi_row4(float4 a4, ResidT res, float b0, float 
     *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
   } else {
     uint2 o;
-    o.x = e_pack2<H>(v[0], v[1]);
-    o.y = e_pack2<H>(v[2], v[3]);
+    o.x = pack2(v[0], v[1]);
+    o.y = pack2(v[2], v[3]);
     *reinterpret_cast<uint2*>(dst) = o;
   }
 }
 
-// QB = 0: bf16 weights, DMA'd like the activations. QB = 4 / 8 (affine) and QMX8 (mxfp8): each
-// stage DMAs the packed weight bytes and the scale (/ bias) words of its group, and every wave
+// QB = 4 / 8 (affine) and QMX8 (mxfp8): each stage DMAs the activations, the packed weight bytes and the scale (/ bias) words of its group, and every wave
 // dequantizes its own weight fragments in registers (bit-exact, the arithmetic of dequant8)
 // between the MFMAs of the previous k16 step: the stage's weights cross LDS once, packed, and no
 // bf16 copy of them is written. TL: the affine weights are in the tiled layout (one contiguous
 // block per 256-row tile and stage, see kx_qweight_tile_affine), else in the reference layout
 // (one 16- or 32-byte piece per row).
-template <int BM, int BN, int QB, bool TL, int GMODE, bool OUTF32, bool NR = false, bool H = false>
+template <int BM, int BN, int QB, bool TL, int GMODE, bool OUTF32>
 __global__ __launch_bounds__(256) void gemm_lds_kernel(
-    const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ W, int64_t ldw,
-    QuantW qw, void* __restrict__ C, int64_t ldc, int M, int N, int K, Epilogue epi) {
-  // stage geometry: dense products, 64-wide stages, in a 2-stage ring for the 256 x 256 and
-  // 192 x 256 tiles and a 4-stage ring for the small tiles (whose few MFMAs per stage cannot
-  // cover a one-stage prefetch); quantized products, 32-wide stages in a 4-stage ring. A row's
-  // 16-byte slots are XOR-swizzled (by (r >> 1) & 7, resp. (r >> 2) & 3) so that the DMA writes
-  // and the 32-row fragment reads are bank-conflict free.
-  constexpr bool D64 = QB == 0;
-  constexpr bool RING2 = D64 && BM * BN >= 192 * 256;
-  constexpr int DBK = D64 ? DENSE_BK : 32;  // K per LDS stage
+    const uint16_t* __restrict__ A, int64_t lda, QuantW qw, void* __restrict__ C, int64_t ldc, int M, int N, int K, Epilogue epi) {
+  // stage geometry: 32-wide stages in a 4-stage ring; a row's 16-byte slots are XOR-swizzled (by
+  // (r >> 2) & 3) so that the DMA writes and the 32-row fragment reads are bank-conflict free
+  constexpr int DBK = 32;                   // K per LDS stage
   constexpr int DROW = DBK * 2;             // bytes per LDS row
   constexpr int DCPR = DBK / 8;             // 16-byte chunks per row
   constexpr int DRPI = 64 / DCPR;           // rows one DMA instruction fills
-  constexpr int DNS = RING2 ? 2 : 4;        // stages in the ring
-  const auto dswz = [](int r) { return D64 ? (r >> 1) & 7 : (r >> 2) & 3; };
+  constexpr int DNS = 4;                    // stages in the ring
+  const auto dswz = [](int r) { return (r >> 2) & 3; };
   constexpr int A_INST = BM / DRPI / 4;
   constexpr int QROW = DBK * qbits<QB>() / 8;                         // packed bytes per row
-  constexpr int WQ_INST = QB ? BN * QROW / 1024 / 4 : 0;              // packed words, per wave
+  constexpr int WQ_INST = BN * QROW / 1024 / 4;                       // packed words, per wave
   constexpr int SB_BYTES = QB == QMX8 ? 4 : 8;                        // scale (bias) bytes per row
-  constexpr int SB_INST = QB ? SB_BYTES * BN / 256 / 4 : 0;           // scale and bias pairs
-  constexpr int W_INST = QB ? WQ_INST + SB_INST : BN / DRPI / 4;
+  constexpr int SB_INST = SB_BYTES * BN / 256 / 4;                    // scale and bias pairs
+  constexpr int W_INST = WQ_INST + SB_INST;
   constexpr int PER = A_INST + W_INST;  // DMA instructions per wave per stage
-  constexpr int W_BYTES = QB ? BN * QROW + BN * SB_BYTES : BN * DROW;
+  constexpr int W_BYTES = BN * QROW + BN * SB_BYTES;
   constexpr int STAGE = BM * DROW + W_BYTES;
   constexpr int RING = DNS * STAGE;
-  // wave layout: dense products 2 x 2 waves of (BM / 2) x (BN / 2); quantized weights 1 x 4 waves
-  // of BM x (BN / 4), so that each weight column is dequantized by one wave only (a 2 x 2 layout
-  // dequantizes every column twice) for the same LDS fragment traffic per MFMA as the dense form
-  constexpr int WGM = QB ? 1 : 2, WGN = 4 / WGM;
+  // wave layout: 1 x 4 waves of BM x (BN / 4), so that each weight column is dequantized by one wave
+  // only (a 2 x 2 layout dequantizes every column twice) for the same LDS fragment traffic per MFMA
+  constexpr int WGM = 1, WGN = 4;
   constexpr int WT_M = BM / WGM, WT_N = BN / WGN;
   constexpr int MB = WT_M / 32, NB = WT_N / 32;
   constexpr int KS = DBK / 16;
-  static_assert(KS == (D64 ? 4 : 2), "k16 steps per stage");
   constexpr int DPS = (PER + KS - 1) / KS;  // DMA instructions per k16 step
   // At the wait in the last k16 step, stages kt+2 .. kt+NS-2 and the DMA of this iteration's
   // earlier steps may stay in flight: stage kt+1 is then complete.
   constexpr int NBEFORE = (KS - 1) * DPS < PER ? (KS - 1) * DPS : PER;
-  constexpr int WAITN = RING2 ? 0 : (DNS - 3) * PER + NBEFORE;
+  constexpr int WAITN = (DNS - 3) * PER + NBEFORE;
   constexpr int PITCH = WT_N / 2 + 4;  // staged epilogue row, floats
   constexpr int EP_BYTES = 4 * WT_M * PITCH * 4;
   constexpr int SMEM = RING > EP_BYTES ? RING : EP_BYTES;
   static_assert(A_INST * DRPI * 4 == BM && MB >= 1 && NB >= 2, "tile");
-  static_assert(QB == 0 ? (BN / DRPI / 4) * DRPI * 4 == BN : (BN == 256 && WQ_INST >= 1), "weight tile");
+  static_assert(BN == 256 && WQ_INST >= 1, "weight tile");
   static_assert(MB + NB <= 15 && WAITN >= 0, "pipeline");
   static_assert(!(TL && QB == QMX8), "mxfp8 weights are read in the reference layout only");
-  static_assert(!H || (QB == 0 && !NR), "fp16 operands: the dense product without the norm epilogue");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[SMEM];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WGM, wn = wave / WGM;
   const int lrow = lane & 31, lhalf = lane >> 5;
-  if constexpr (QB == 0 && GMODE == 0 && OUTF32) {
-    // split-K (grid.y > 1): workgroup row y multiplies K slice y (K is the slice length) and
-    // writes its fp32 partial product to plane y of C (planes M * ldc floats apart)
-    const int64_t y = blockIdx.y;
-    A += y * K;
-    W += y * K;
-    C = static_cast<float*>(C) + y * (int64_t)M * ldc;
-  }
 
   // tile coordinates (see lds_tile_of)
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
@@ -735,18 +541,11 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
     vo[i] = (uint32_t)(((int64_t)(min(m0 + r, M - 1) - m0) * lda + (slot ^ dswz(r)) * 8) * 2);
   }
   const char* a_base = reinterpret_cast<const char*>(A + (int64_t)m0 * lda);
-  const char* w_base;   // bf16 weights, or the packed words
+  const char* w_base;            // the packed words
   const char* s_base = nullptr;  // scale pairs (bias pairs follow at b_base)
   const char* b_base = nullptr;
   const int64_t qrow_bytes = (int64_t)K * qbits<QB>() / 8, groups = K / 64;
-  if constexpr (QB == 0) {
-#pragma unroll
-    for (int i = 0; i < W_INST; ++i) {
-      const int r = (wave * W_INST + i) * DRPI + r_in;
-      vo[A_INST + i] = (uint32_t)(((int64_t)(min(n0 + r, N - 1) - n0) * ldw + (slot ^ dswz(r)) * 8) * 2);
-    }
-    w_base = reinterpret_cast<const char*>(W + (int64_t)n0 * ldw);
-  } else if constexpr (TL) {
+  if constexpr (TL) {
     // tiled: the stage's packed words (BN * QROW bytes) and scale / bias pairs (BN * 8 bytes of
     // its 128-wide window) are contiguous blocks (8-bit rows: chunk swizzle as below)
 #pragma unroll
@@ -787,14 +586,12 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
       b_base = reinterpret_cast<const char*>(qw.biases) + (int64_t)n0 * sb_row;
     }
   }
-  // dense operands: buffer loads (the tile bases as resources; lane offsets < 2^31, K offsets
-  // < 2^23 by the dispatch's stride limits)
-  const rsrc_t a_rsrc = raw_rsrc(a_base), w_rsrc = raw_rsrc(w_base);
+  // activations: buffer loads (the tile base as the resource; lane offsets < 2^31, K offsets < 2^23
+  // by the dispatch's stride limits)
+  const rsrc_t a_rsrc = raw_rsrc(a_base);
   auto dma = [&](int i, uint8_t* buf, int k0) {
     if (i < A_INST) {
       buffer_lds16(a_rsrc, buf + (wave * A_INST + i) * DRPI * DROW, vo[i], (uint32_t)k0 * 2);
-    } else if constexpr (QB == 0) {
-      buffer_lds16(w_rsrc, buf + (BM + (wave * W_INST + i - A_INST) * DRPI) * DROW, vo[i], (uint32_t)k0 * 2);
     } else if (TL && i < A_INST + WQ_INST) {
       __builtin_amdgcn_global_load_lds((const void*)(w_base + (int64_t)(k0 / DBK) * (BN * QROW) + vo[i]),
                                        KX_LDS(buf + BM * DROW + (wave * WQ_INST + i - A_INST) * 1024), 16, 0, 0);
@@ -818,33 +615,18 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
     }
   };
 
-  // fragment byte offsets, per k16 step (the MFMA A operand is the weight tile). Dense: step s
-  // of lane half h covers k = 16 s + 8 h .. + 7 of the stage. Quantized: k = 16 h + 8 s .. + 7
-  // (the same permutation of the sum on both operands), so that a lane's packed weight bytes of
-  // both steps are contiguous and come in one read per stage.
-  int a_off[KS][MB], w_off[KS][NB];
+  // fragment byte offsets, per k16 step (the MFMA A operand is the weight tile): step s of lane
+  // half h covers k = 16 h + 8 s .. + 7 of the stage (the same permutation of the sum on both
+  // operands), so that a lane's packed weight bytes of both steps are contiguous and come in one
+  // read per stage
+  int a_off[KS][MB];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    const int c = QB ? 2 * lhalf + s : 2 * s + lhalf;
+  for (int s = 0; s < KS; ++s)
 #pragma unroll
     for (int j = 0; j < MB; ++j) {
-      const int r = wm * WT_M + j * 32 + lrow;
-      a_off[s][j] = r * DROW + ((c ^ dswz(r)) << 4);
+      const int r = j * 32 + lrow;
+      a_off[s][j] = r * DROW + (((2 * lhalf + s) ^ dswz(r)) << 4);
     }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int r = wn * WT_N + i * 32 + lrow;
-      w_off[s][i] = BM * DROW + r * DROW + ((c ^ dswz(r)) << 4);
-    }
-  }
-  auto load_frags = [&](const uint8_t* buf, int s, bf16x8* af, bf16x8* wf) {
-#pragma unroll
-    for (int j = 0; j < MB; ++j) af[j] = *reinterpret_cast<const bf16x8*>(buf + a_off[s][j]);
-    if constexpr (QB == 0) {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) wf[i] = *reinterpret_cast<const bf16x8*>(buf + w_off[s][i]);
-    }
-  };
 
   f32x16 acc[NB][MB];
 #pragma unroll
@@ -855,27 +637,16 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
   const int stages = K / DBK;
-  // dense: stage 0, and the first DH1 DMA instructions of stage 1 (the rest go out in stage 0's
-  // first step); quantized: stages 0 .. NS-2
-  constexpr int DH1 = (PER + 1) / 2;
-  if constexpr (RING2) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) dma(i, smem, 0);
+  for (int p = 0; p < DNS - 1; ++p)
 #pragma unroll
-    for (int i = 0; i < DH1; ++i) dma(i, smem + STAGE, min(1, stages - 1) * DBK);
-    wait_vmcnt<DH1>();
-  } else {
-#pragma unroll
-    for (int p = 0; p < DNS - 1; ++p)
-#pragma unroll
-      for (int i = 0; i < PER; ++i) dma(i, smem + p * STAGE, min(p, stages - 1) * DBK);
-    wait_vmcnt<(DNS - 2) * PER>();
-  }
+    for (int i = 0; i < PER; ++i) dma(i, smem + p * STAGE, min(p, stages - 1) * DBK);
+  wait_vmcnt<(DNS - 2) * PER>();
   KX_BARRIER();
   bf16x8 fa[2][MB], fw[2][NB];
   int cur_i = 0;
-  if constexpr (QB != 0) {
-    // ---- quantized mainloop: every wave dequantizes its own weight fragments in registers ----
+  {
+    // ---- mainloop: every wave dequantizes its own weight fragments in registers ----
     // A lane's packed bytes of weight block i for the whole stage (both k16 steps of its row)
     // and the row's scale (and bias) word; read once per stage, right after the stage's barrier.
     using Raw = typename std::conditional<qbits<QB>() == 4, uint2, uint4>::type;
@@ -992,7 +763,7 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
 #pragma unroll
       for (int q = 0; q < NMF; ++q) {
         const int i = q / MB, j = q % MB;
-        acc[i][j] = mfma32x32x16<H>(fw[0][i], fa[0][j], acc[i][j]);
+        acc[i][j] = mfma32x32x16<false>(fw[0][i], fa[0][j], acc[i][j]);
         if (q < MB) fa[1][q] = *reinterpret_cast<const bf16x8*>(cur + a_off[1][q]);
         if (q < DPS && q < PER) dma(q, iss, k_iss);
 #pragma unroll
@@ -1012,7 +783,7 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
 #pragma unroll
       for (int q = 0; q < QSPLIT; ++q) {
         const int i = q / MB, j = q % MB;
-        acc[i][j] = mfma32x32x16<H>(fw[1][i], fa[1][j], acc[i][j]);
+        acc[i][j] = mfma32x32x16<false>(fw[1][i], fa[1][j], acc[i][j]);
 #pragma unroll
         for (int r = q * NRD1 / QSPLIT; r < (q + 1) * NRD1 / QSPLIT; ++r) stage_read(r, nxt);
 #pragma unroll
@@ -1026,7 +797,7 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
 #pragma unroll
       for (int q = QSPLIT; q < NMF; ++q) {
         const int i = q / MB, j = q % MB;
-        acc[i][j] = mfma32x32x16<H>(fw[1][i], fa[1][j], acc[i][j]);
+        acc[i][j] = mfma32x32x16<false>(fw[1][i], fa[1][j], acc[i][j]);
 #pragma unroll
         for (int idx = (q - QSPLIT) * NPAIR / (NMF - QSPLIT); idx < (q - QSPLIT + 1) * NPAIR / (NMF - QSPLIT); ++idx)
           dq_step(idx, 0);
@@ -1035,124 +806,8 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
       dq_commit(fw[0]);
       cur_i = nxt_i;
     }
-  } else if constexpr (!RING2) {
-    load_frags(smem, 0, fa[0], fw[0]);
-    for (int kt = 0; kt < stages; ++kt) {
-      const uint8_t* cur = smem + cur_i * STAGE;
-      const int nxt_i = cur_i + 1 == DNS ? 0 : cur_i + 1;
-      // stage kt+NS-1 goes into the buffer stage kt-1 used; past the end the last stage is
-      // re-read into it, which keeps the loop free of branches and the vmcnt arithmetic uniform
-      uint8_t* iss = smem + (cur_i == 0 ? DNS - 1 : cur_i - 1) * STAGE;
-      const int k_iss = min(kt + DNS - 1, stages - 1) * DBK;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const int b = s & 1;
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkmcnt0();
-        if (s + 1 == KS) {
-          // stage kt+1 has landed for this wave and its reads of cur are done; after the barrier
-          // this holds for every wave, and nobody reads cur again before it is refilled
-          wait_vmcnt<WAITN>();
-          KX_BARRIER();
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        // after each MFMA, its share of the next step's fragment reads (after the last step:
-        // stage kt+1's first) and of this step's DMA issues, in source order
-        const uint8_t* rbuf = s + 1 < KS ? cur : smem + nxt_i * STAGE;
-        const int rs = s + 1 < KS ? s + 1 : 0;
-        constexpr int NRD = MB + NB, NMF = NB * MB;
-        const int d0 = s * DPS, nd = PER - d0 < DPS ? (PER - d0 > 0 ? PER - d0 : 0) : DPS;
-#pragma unroll
-        for (int q = 0; q < NMF; ++q) {
-          const int i = q / MB, j = q % MB;
-          acc[i][j] = mfma32x32x16<H>(fw[b][i], fa[b][j], acc[i][j]);
-#pragma unroll
-          for (int r = q * NRD / NMF; r < (q + 1) * NRD / NMF; ++r) {
-            if (r < MB) {
-              fa[b ^ 1][r] = *reinterpret_cast<const bf16x8*>(rbuf + a_off[rs][r]);
-            } else {
-              fw[b ^ 1][r - MB] = *reinterpret_cast<const bf16x8*>(rbuf + w_off[rs][r - MB]);
-            }
-          }
-#pragma unroll
-          for (int d = q * nd / NMF; d < (q + 1) * nd / NMF; ++d) dma(d0 + d, iss, k_iss);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      cur_i = nxt_i;
-    }
-  } else {
-    // Two 64-wide stages. Stage kt+2 goes into stage kt's buffer: its first DH1 DMA instructions
-    // right after the barrier of stage kt's last k16 step (every wave has read that buffer's
-    // last fragments by then), the rest during step 0 of stage kt+1; the barrier of stage
-    // kt+1's last step waits for all of them. Past the end the last stage is re-read, which
-    // keeps the loop free of branches and the vmcnt arithmetic uniform. Each MFMA is followed by
-    // its share of the fragment reads and DMA issues, in source order (the compiler's own
-    // placement bunched the DMA issues, ~10 VALU / SALU / VMEM instructions each, between two
-    // MFMAs and left the matrix core idle: 5 % on every block shape).
-    load_frags(smem, 0, fa[0], fw[0]);
-    for (int kt = 0; kt < stages; ++kt) {
-      uint8_t* cur = smem + (kt & 1) * STAGE;
-      uint8_t* oth = smem + ((kt & 1) ^ 1) * STAGE;
-      const int k1 = min(kt + 1, stages - 1) * DBK;
-      const int k2 = min(kt + 2, stages - 1) * DBK;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const int b = s & 1;
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lgkmcnt0();
-        if (s + 1 == KS) {
-          wait_vmcnt<0>();
-          KX_BARRIER();
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        // the next step's fragments (after the last step: stage kt+1's first) and this step's
-        // DMA issues, one group after each MFMA, in a fixed order
-        const uint8_t* rbuf = s + 1 < KS ? cur : oth;
-        const int rs = s + 1 < KS ? s + 1 : 0;
-        constexpr int NRD = MB + NB, NMF = NB * MB;
-        const int nd = s == 0 ? PER - DH1 : s + 1 == KS ? DH1 : 0;
-        const int d0 = s == 0 ? DH1 : 0;
-        uint8_t* dbuf = s == 0 ? oth : cur;
-        const int dk = s == 0 ? k1 : k2;
-#pragma unroll
-        for (int q = 0; q < NMF; ++q) {
-          const int i = q / MB, j = q % MB;
-          acc[i][j] = mfma32x32x16<H>(fw[b][i], fa[b][j], acc[i][j]);
-          if (q < MB) {
-            fa[b ^ 1][q] = *reinterpret_cast<const bf16x8*>(rbuf + a_off[rs][q]);
-          } else if (q < NRD) {
-            fw[b ^ 1][q - MB] = *reinterpret_cast<const bf16x8*>(rbuf + w_off[rs][q - MB]);
-          }
-#pragma unroll
-          for (int d = q * nd / NMF; d < (q + 1) * nd / NMF; ++d) dma(d0 + d, dbuf, dk);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    }
   }
   wait_vmcnt<0>();
-
-  // ---- KX_EPI_QK_NORM_ROPE (NR): a wave's 128 columns are one head. A query or key head's wave
-  // stages its two halves twice: the first time its store-loop lanes sum the squares of bias +
-  // accumulator, rounded to bf16 as the projection's output would be, over their rows (each
-  // row's 128 columns spread over 16 lanes and both halves), the second time they apply the
-  // same rounded values' weighted RMSNorm and the adjacent-pair rotation in fp32
-  // (each product of the rotation rounded before the sum, as the standalone norm + RoPE kernel
-  // does) and store. Reading the accumulators only through the staging keeps them in place.
-  bool bias_done = false;  // a norm wave: its store loop adds the bias
-  int64_t nr_head = 0;
-  const void* nr_w = nullptr;
-  if constexpr (NR) {
-    static_assert(WT_N == 128 && GMODE == 0 && !OUTF32 && QB == 0, "one 128-wide head per wave");
-    const int64_t ncol0 = (int64_t)n0 + wn * WT_N;
-    if (ncol0 < epi.k_end) {
-      const bool isq = ncol0 < epi.q_end;
-      nr_w = isq ? epi.nq : epi.nk;
-      nr_head = isq ? ncol0 / 128 : (ncol0 - epi.q_end) / 128;
-      bias_done = true;
-    }
-  }
 
   // ---- epilogue: the accumulator lane holds row m = j*32 + lrow and columns 8g + 4 lhalf + e of
   // block i; staged per half of the wave's columns into a private LDS region.
@@ -1166,29 +821,10 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
   const int act = (epi.flags >> 4) & 15;
   const bool has_bias = epi.flags & KX_EPI_BIAS;
   const int mrow0 = m0 + wm * WT_M;
-  // Full tiles read the residual of all of a lane's rows of a half before any compute or store:
-  // the loads are in flight together (C may alias the residual, so loads issued after a store
-  // would wait for it), and the half's LDS staging and barrier run under their latency.
-  constexpr int NROW = WT_M / RPI_EP;  // rows per lane per half
-  static_assert(NROW * RPI_EP == WT_M, "epilogue rows");
-  // residual rows are prefetched in chunks of PF rows. 256-row tiles hold all 256 accumulator
-  // registers through the epilogue and have no room for the prefetch: they read the residual
-  // row by row (PREF false); so do the 1 x 4 quantized layouts, whose lanes hold 192 or 256 rows.
-  constexpr bool PREF = GMODE != 0 && BM <= 192 && WGM == 2;
-  constexpr int PF = NROW > 24 ? NROW / 2 : NROW;
-  constexpr int NCH = NROW / PF;
-  static_assert(NCH * PF == NROW && PF % 4 == 0, "epilogue chunks");
   using ResidT = typename std::conditional<GMODE == 2, float4, uint2>::type;
-  ResidT rpre[PREF ? PF : 1];
   const int64_t resid_es = GMODE == 2 ? 4 : 2;
   const char* rbase = GMODE == 0 ? nullptr
       : reinterpret_cast<const char*>(epi.resid) + ((int64_t)mrow0 * epi.ldr + n0 + wn * WT_N + 4 * q) * resid_es;
-#define KX_PREFETCH_RESID(h, c)                                                                    \
-  _Pragma("unroll") for (int k = 0; k < PF; ++k) rpre[k] = *reinterpret_cast<const ResidT*>(       \
-      rbase + ((int64_t)(rr + ((c) * PF + k) * RPI_EP) * epi.ldr + (h) * HALF_N) * resid_es);
-  if constexpr (PREF) {
-    if (full) { KX_PREFETCH_RESID(0, 0) }
-  }
   KX_BARRIER();  // every wave is done with the main loop's LDS
   // The half loop is not unrolled (its body is large); each half stages its accumulator blocks
   // under its own branch so that every accumulator index stays a compile-time constant.
@@ -1197,16 +833,8 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
   _Pragma("unroll") for (int g = 0; g < 4; ++g)                                                   \
       *reinterpret_cast<float4*>(ep + (j * 32 + lrow) * PITCH + (ii) * 32 + 8 * g + 4 * lhalf) =  \
           make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-  float nr_ss[NR ? NROW : 1], nr_inv[NR ? NROW : 1];  // NR: per row of this lane
-#pragma unroll
-  for (int k = 0; k < (NR ? NROW : 1); ++k) nr_ss[k] = 0.0f;
-  const int passes = NR && bias_done ? 4 : 2;  // norm waves: two summing passes, then two storing
 #pragma unroll 1
-  for (int hp = 0; hp < passes; ++hp) {
-    const int h = hp & 1;
-    if constexpr (PREF) {
-      if (h == 1 && full) { KX_PREFETCH_RESID(1, 0) }
-    }
+  for (int h = 0; h < 2; ++h) {
     if (h == 0) {
 #pragma unroll
       for (int ii = 0; ii < NB / 2; ++ii) { KX_STAGE_BLOCK(ii, ii) }
@@ -1217,116 +845,12 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
 #undef KX_STAGE_BLOCK
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const int n = n0 + wn * WT_N + h * HALF_N + 4 * q;
-    if (NR && bias_done && hp < 2) {
-      // summing pass: this lane's 4 columns of each of its rows
-      float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (has_bias) {
-        const uint2 bb = *reinterpret_cast<const uint2*>(epi.bias + n);
-        b4[0] = e_lo<H>(bb.x); b4[1] = e_hi<H>(bb.x); b4[2] = e_lo<H>(bb.y); b4[3] = e_hi<H>(bb.y);
-      }
-#pragma unroll
-      for (int k = 0; k < (NR ? NROW : 1); ++k) {
-        const float4 a4 = *reinterpret_cast<const float4*>(ep + (rr + k * RPI_EP) * PITCH + 4 * q);
-        const float v0 = bf2f(f2bf(a4.x + b4[0])), v1 = bf2f(f2bf(a4.y + b4[1]));
-        const float v2 = bf2f(f2bf(a4.z + b4[2])), v3 = bf2f(f2bf(a4.w + b4[3]));
-        nr_ss[k] = fmaf(v3, v3, fmaf(v2, v2, fmaf(v1, v1, fmaf(v0, v0, nr_ss[k]))));
-      }
-      if (hp == 1) {
-        // a row's 16 lanes (lane / LPR is the row slot) add their sums; then 1 / rms
-#pragma unroll
-        for (int k = 0; k < (NR ? NROW : 1); ++k) {
-          static_assert(!NR || LPR == 16, "a staged row's lanes are one DPP row");
-          nr_inv[k] = rsqrtf(row16_sum(nr_ss[k]) * (1.0f / 128.0f) + epi.n_eps);
-        }
-      }
-    } else if (NR && bias_done) {
-      // storing pass: bias, norm and rotation of 4 columns per lane of a query / key head (whole
-      // inside N)
-      const int d = h * HALF_N + 4 * q;  // column within the head; pairs (d, d+1), (d+2, d+3)
-      float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w4[4];
-      if (has_bias) {
-        const uint2 bb = *reinterpret_cast<const uint2*>(epi.bias + n);
-        b4[0] = e_lo<H>(bb.x); b4[1] = e_hi<H>(bb.x); b4[2] = e_lo<H>(bb.y); b4[3] = e_hi<H>(bb.y);
-      }
-      if (epi.n_bf16) {
-        const uint2 ww = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(nr_w) + d);
-        w4[0] = lo_f(ww.x); w4[1] = hi_f(ww.x); w4[2] = lo_f(ww.y); w4[3] = hi_f(ww.y);
-      } else {
-        const float4 ww = *reinterpret_cast<const float4*>(static_cast<const float*>(nr_w) + d);
-        w4[0] = ww.x; w4[1] = ww.y; w4[2] = ww.z; w4[3] = ww.w;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) w4[e] += epi.n_off;
-      // Rows go in groups of GR: the group's table rows (a row clamped to M - 1 past the end) are
-      // loaded together, so one memory latency covers GR rows. Table row of output row m: m / t_rows
-      // by the host's magic number (m < 2^31: umulhi(m, magic) + m fits 32 bits).
-      if constexpr (NR) {
-        constexpr int GR = 8, NG = NROW / GR;
-        static_assert(NROW % GR == 0, "NR row groups");
-        const float* ct = epi.cosp + nr_head * epi.t_hs + d;
-        const float* st = epi.sinp + nr_head * epi.t_hs + d;
-        const uint32_t t_rows = (uint32_t)epi.t_rows, t_bs = (uint32_t)epi.t_bs, t_ld = (uint32_t)epi.t_ld;
-        // the rows' offsets are the same in both storing passes: opaque here, so that they are
-        // computed per pass and group rather than held in registers across the epilogue
-        int mb = mrow0 + rr;
-        asm volatile("" : "+v"(mb));
-        uint16_t* crow = static_cast<uint16_t*>(C) + (int64_t)mb * ldc + n;
-        // two groups of table rows in flight: group g + 1's loads are issued before group g's math
-        float4 c4[2][GR], s4[2][GR];
-        auto load_group = [&](int g0, float4* cg, float4* sg) {
-#pragma unroll
-          for (int j = 0; j < GR; ++j) {
-            const uint32_t m = (uint32_t)min(mb + (g0 + j) * RPI_EP, M - 1);
-            const uint32_t seq = (__umulhi(m, epi.t_magic) + m) >> epi.t_shift;
-            const uint32_t trow = seq * t_bs + (m - seq * t_rows) * t_ld;  // < 2^31 (host check)
-            cg[j] = *reinterpret_cast<const float4*>(ct + trow);
-            sg[j] = *reinterpret_cast<const float4*>(st + trow);
-          }
-        };
-        load_group(0, c4[0], s4[0]);
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi) {
-          if (gi + 1 < NG) load_group((gi + 1) * GR, c4[(gi + 1) & 1], s4[(gi + 1) & 1]);
-          const float4* cg = c4[gi & 1];
-          const float4* sg = s4[gi & 1];
-#pragma unroll
-          for (int j = 0; j < GR; ++j) {
-            const int k = gi * GR + j;
-            const int r = rr + k * RPI_EP;
-            const int m = mb + k * RPI_EP;
-            const float4 a4 = *reinterpret_cast<const float4*>(ep + r * PITCH + 4 * q);
-            const float iv = nr_inv[k];
-            const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-            const float c[4] = {cg[j].x, cg[j].y, cg[j].z, cg[j].w}, sn[4] = {sg[j].x, sg[j].y, sg[j].z, sg[j].w};
-            float nv[4], o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) nv[e] = bf2f(f2bf(av[e] + b4[e])) * iv * w4[e];
-#pragma unroll
-            for (int e = 0; e < 4; e += 2) {
-#pragma clang fp contract(off)
-              const float a0 = nv[e] * c[e];
-              const float b0 = (-nv[e + 1]) * sn[e];
-              const float a1 = nv[e + 1] * c[e + 1];
-              const float b1 = nv[e] * sn[e + 1];
-              o[e] = a0 + b0;
-              o[e + 1] = a1 + b1;
-            }
-            uint2 sv;
-            sv.x = pack2(o[0], o[1]);
-            sv.y = pack2(o[2], o[3]);
-            if (m < M) *reinterpret_cast<uint2*>(crow + (int64_t)(k * RPI_EP) * ldc) = sv;
-          }
-          // keeps group g + 2's loads (and their address arithmetic) below this group's math
-          asm volatile("" ::: "memory");
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    } else if (full) {
+    if (full) {
       // column data is fixed per lane: bias, and the gate when one gate row covers the rows
       float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       if (has_bias) {
         const uint2 bb = *reinterpret_cast<const uint2*>(epi.bias + n);
-        b4[0] = e_lo<H>(bb.x); b4[1] = e_hi<H>(bb.x); b4[2] = e_lo<H>(bb.y); b4[3] = e_hi<H>(bb.y);
+        b4[0] = lo_f(bb.x); b4[1] = hi_f(bb.x); b4[2] = lo_f(bb.y); b4[3] = hi_f(bb.y);
       }
       const int64_t gstride = epi.gate_stride, gdiv = epi.gate_div;
       const bool gate_const = GMODE == 0 || gstride == 0 || (mrow0 / gdiv) == ((mrow0 + WT_M - 1) / gdiv);
@@ -1338,48 +862,19 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
       auto full_rows = [&](auto act_tag, auto gate_tag) {
         constexpr int ACT = decltype(act_tag)::value;
         constexpr bool GC = decltype(gate_tag)::value;  // one gate row covers the wave's rows
-        if constexpr (!PREF) {
 #pragma unroll 4
-          for (int r = rr; r < WT_M; r += RPI_EP) {
-            ResidT res{};
-            float4 gv = g4c;
-            if constexpr (GMODE != 0) {
-              res = *reinterpret_cast<const ResidT*>(rbase + ((int64_t)r * epi.ldr + h * HALF_N) * resid_es);
-              if constexpr (!GC) {
-                const int64_t grow = gdiv == 1 ? (int64_t)(mrow0 + r) : (int64_t)(mrow0 + r) / gdiv;
-                gv = *reinterpret_cast<const float4*>(epi.gate + grow * gstride + n);
-              }
-            }
-            epi_row4<H, GMODE, OUTF32, ACT>(*reinterpret_cast<const float4*>(ep + r * PITCH + 4 * q), res, b4[0],
-                                         b4[1], b4[2], b4[3], act, gv, cbase + (int64_t)r * ldc * (OUTF32 ? 4 : 2));
-          }
-        } else {
-          // groups of 4 rows: their staged reads together, then their stores (bounded registers:
-          // the prefetched residual stays live, the staged values of one group at a time)
-          constexpr int GR = 4;
-#pragma unroll
-          for (int c = 0; c < NCH; ++c) {
-            if (c > 0) { KX_PREFETCH_RESID(h, c) }
-#pragma unroll
-            for (int k0 = 0; k0 < PF; k0 += GR) {
-              float4 a4[GR];
-#pragma unroll
-              for (int k = 0; k < GR; ++k)
-                a4[k] = *reinterpret_cast<const float4*>(ep + (rr + (c * PF + k0 + k) * RPI_EP) * PITCH + 4 * q);
-#pragma unroll
-              for (int k = 0; k < GR; ++k) {
-                const int r = rr + (c * PF + k0 + k) * RPI_EP;
-                float4 gv = g4c;
-                if constexpr (!GC) {
-                  const int64_t grow = gdiv == 1 ? (int64_t)(mrow0 + r) : (int64_t)(mrow0 + r) / gdiv;
-                  gv = *reinterpret_cast<const float4*>(epi.gate + grow * gstride + n);
-                }
-                epi_row4<H, GMODE, OUTF32, ACT>(a4[k], rpre[k0 + k], b4[0], b4[1], b4[2], b4[3], act, gv,
-                                             cbase + (int64_t)r * ldc * (OUTF32 ? 4 : 2));
-              }
-              __builtin_amdgcn_sched_barrier(0);
+        for (int r = rr; r < WT_M; r += RPI_EP) {
+          ResidT res{};
+          float4 gv = g4c;
+          if constexpr (GMODE != 0) {
+            res = *reinterpret_cast<const ResidT*>(rbase + ((int64_t)r * epi.ldr + h * HALF_N) * resid_es);
+            if constexpr (!GC) {
+              const int64_t grow = gdiv == 1 ? (int64_t)(mrow0 + r) : (int64_t)(mrow0 + r) / gdiv;
+              gv = *reinterpret_cast<const float4*>(epi.gate + grow * gstride + n);
             }
           }
+          epi_row4<GMODE, OUTF32, ACT>(*reinterpret_cast<const float4*>(ep + r * PITCH + 4 * q), res, b4[0],
+                                       b4[1], b4[2], b4[3], act, gv, cbase + (int64_t)r * ldc * (OUTF32 ? 4 : 2));
         }
       };
       using Const = std::true_type;
@@ -1396,13 +891,12 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
         const float4 a4 = *reinterpret_cast<const float4*>(ep + r * PITCH + 4 * q);
         if (m < M && n < N) {
           float v[4] = {a4.x, a4.y, a4.z, a4.w};
-          epilogue_store4<H>(v, m, n, N, epi, C, ldc, vec_ok);
+          epilogue_store4<false>(v, m, n, N, epi, C, ldc, vec_ok);
         }
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
-#undef KX_PREFETCH_RESID
 }
 
 // ---- skinny kernel (N <= 64: the gate-logit projections) ------------------------------------
@@ -1418,15 +912,6 @@ __global__ __launch_bounds__(256) void gemm_lds_kernel(
 // row) instead of the 32 rows of a 32x32x16 operand, which halves the cache lines each load
 // instruction touches, the limit of this kernel.
 // Quantized weights are dequantized in registers with the arithmetic of the other kernels.
-// One 16x16x32 MFMA on 16-bit operands (bf16, or fp16 with H).
-template <bool H>
-__device__ __forceinline__ f32x4 mfma16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
-  if constexpr (H)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
 template <int QB, int NWK, int RB, bool H = false>
 __global__ __launch_bounds__(NWK * 64) void gemm_skinny_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ W, int64_t ldw,
@@ -1692,67 +1177,38 @@ int pick_cfg(int64_t m, int64_t n) {
   return T128x128;
 }
 
-// Whether a product visits its tile rows last to first. Every producer of an activation in
-// this library writes its rows in ascending order, so the last rows written are the ones most
-// likely still in the 256 MB memory-side cache. When the input is too large for that cache to
-// hold whole (above 128 MiB: the 9216 x 16384 feed-forward hidden state, 302 MB, read by the
-// down projection right after the up projection wrote it), reading its rows newest first turns
-// part of the operand stream into cache hits (down projection 964 -> 927 us in the config-3
-// block). The order of tiles does not change any result.
-bool rows_last_first(int64_t m, int64_t k) { return m * k * 2 > (128ll << 20); }
-
-template <int BM, int BN, int QB, bool TL, int GMODE, bool OUTF32, bool NR = false, bool H = false>
-int launch_lds_t(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, QuantW qw, void* c,
-                 int64_t ldc, int m, int n, int k, const Epilogue& epi, hipStream_t s) {
-  const int tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
+template <int BM, int QB, bool TL, int GMODE, bool OUTF32>
+void launch_lds_t(const uint16_t* a, int64_t lda, QuantW qw, void* c, int64_t ldc, int m, int n, int k,
+                  const Epilogue& epi, hipStream_t s) {
+  const int tiles = ((m + BM - 1) / BM) * ((n + 255) / 256);
   Epilogue e = epi;
   e.rows_desc = rows_last_first(m, k);
-  gemm_lds_kernel<BM, BN, QB, TL, GMODE, OUTF32, NR, H><<<tiles, 256, 0, s>>>(a, lda, w, ldw, qw, c, ldc, m, n, k, e);
-  return KX_OK;
+  gemm_lds_kernel<BM, 256, QB, TL, GMODE, OUTF32><<<tiles, 256, 0, s>>>(a, lda, qw, c, ldc, m, n, k, e);
 }
 
 // Residual mode (none / bf16 / fp32) and output type select the epilogue specialisation.
-template <int BM, int BN, int QB, bool TL = false, bool H = false>
-int launch_lds(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, QuantW qw, void* c,
-               int64_t ldc, int m, int n, int k, const Epilogue& epi, hipStream_t s) {
+template <int BM, int QB, bool TL = false>
+void launch_lds(const uint16_t* a, int64_t lda, QuantW qw, void* c, int64_t ldc, int m, int n, int k,
+                const Epilogue& epi, hipStream_t s) {
   const int gmode = (epi.flags & KX_EPI_GATED_RESIDUAL) ? ((epi.flags & KX_EPI_RESID_F32) ? 2 : 1) : 0;
   const bool out32 = epi.flags & KX_EPI_OUT_F32;
   switch (gmode * 2 + (out32 ? 1 : 0)) {
-    case 0: return launch_lds_t<BM, BN, QB, TL, 0, false, false, H>(a, lda, w, ldw, qw, c, ldc, m, n, k, epi, s);
-    case 1: return launch_lds_t<BM, BN, QB, TL, 0, true, false, H>(a, lda, w, ldw, qw, c, ldc, m, n, k, epi, s);
-    case 2: return launch_lds_t<BM, BN, QB, TL, 1, false, false, H>(a, lda, w, ldw, qw, c, ldc, m, n, k, epi, s);
-    case 3: return launch_lds_t<BM, BN, QB, TL, 1, true, false, H>(a, lda, w, ldw, qw, c, ldc, m, n, k, epi, s);
-    case 4: return launch_lds_t<BM, BN, QB, TL, 2, false, false, H>(a, lda, w, ldw, qw, c, ldc, m, n, k, epi, s);
-    default: return launch_lds_t<BM, BN, QB, TL, 2, true, false, H>(a, lda, w, ldw, qw, c, ldc, m, n, k, epi, s);
+    case 0: return launch_lds_t<BM, QB, TL, 0, false>(a, lda, qw, c, ldc, m, n, k, epi, s);
+    case 1: return launch_lds_t<BM, QB, TL, 0, true>(a, lda, qw, c, ldc, m, n, k, epi, s);
+    case 2: return launch_lds_t<BM, QB, TL, 1, false>(a, lda, qw, c, ldc, m, n, k, epi, s);
+    case 3: return launch_lds_t<BM, QB, TL, 1, true>(a, lda, qw, c, ldc, m, n, k, epi, s);
+    case 4: return launch_lds_t<BM, QB, TL, 2, false>(a, lda, qw, c, ldc, m, n, k, epi, s);
+    default: return launch_lds_t<BM, QB, TL, 2, true>(a, lda, qw, c, ldc, m, n, k, epi, s);
   }
 }
 
-// Tile for the direct-to-LDS kernel: the fewest rounds of 256 workgroups, weighted by the
-// tile's relative speed (a bigger tile reuses each LDS byte more). 0: 256x256, 1: 192x256,
-// 2: 128x128.
-int pick_lds_cfg(int64_t m, int64_t n) {
+// Tile height of the quantized direct-to-LDS kernel (256-wide tiles): the fewest rounds of 256
+// workgroups times their rows (KX355_GEMM_LDS_TILE = 0 / 1 forces 256 / 192).
+bool quantized_tall(int64_t m, int64_t n) {
   const char* env = getenv("KX355_GEMM_LDS_TILE");
-  if (env && *env) {
-    const int v = atoi(env);
-    if (v >= 0 && v <= 3) return v;
-  }
-  // tiles 256x256, 192x256, 128x128 and (for a few hundred rows, e.g. the text K/V projection)
-  // 64x128, which fills the CUs where 128x128 leaves half of them idle. Speeds per unit of tile
-  // area relative to 256x256, measured: 192x256 runs 3-5 % slower per FLOP at 9216 and 27 280
-  // rows (it moves 17 % more bytes per FLOP through L2 and LDS)
-  const int64_t bm[4] = {256, 192, 128, 64}, bn[4] = {256, 256, 128, 128};
-  const double speed[4] = {1.0, 0.93, 0.8, 0.6};
-  int best = 0;
-  double best_cost = 0.0;
-  for (int i = 0; i < 4; ++i) {
-    const int64_t tiles = ((m + bm[i] - 1) / bm[i]) * ((n + bn[i] - 1) / bn[i]);
-    const double cost = (double)((tiles + 255) / 256) * (double)(bm[i] * bn[i]) / speed[i];
-    if (i == 0 || cost < best_cost) {
-      best = i;
-      best_cost = cost;
-    }
-  }
-  return best;
+  if (env && (env[0] == '0' || env[0] == '1')) return env[0] == '0';
+  const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t192 = ((m + 191) / 192) * ((n + 255) / 256);
+  return (t256 + 255) / 256 * 256 <= (t192 + 255) / 256 * 192;
 }
 
 template <int QB, bool H = false>
@@ -1765,14 +1221,10 @@ int dispatch(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, Qua
     launch_skinny<QB, H>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
     return KX_OK;
   }
-  // the direct-to-LDS kernel keeps per-lane 32-bit byte offsets within a 256-row tile
+  // the direct-to-LDS kernels keep per-lane 32-bit byte offsets within a 256-row tile
   if (QB == 0 && k % DENSE_BK == 0 && lda <= (1 << 22) && ldw <= (1 << 22) && !use_legacy) {
-    switch (pick_lds_cfg(m, n)) {
-      case 0: return launch_lds<256, 256, 0, false, H>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-      case 1: return launch_lds<192, 256, 0, false, H>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-      case 2: return launch_lds<128, 128, 0, false, H>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-      default: return launch_lds<64, 128, 0, false, H>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-    }
+    launch_dense(H, a, lda, w, ldw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    return KX_OK;
   }
   // quantized weights: the direct-to-LDS kernel with in-LDS dequantization needs whole 128-wide
   // K blocks (scale / bias pairs of two groups), 16-byte aligned packed rows and 4-byte aligned
@@ -1784,12 +1236,13 @@ int dispatch(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, Qua
                                            (reinterpret_cast<uintptr_t>(qw.biases) & 3) == 0;
   if (QB != 0 && k % 128 == 0 && lda <= (1 << 22) && n >= 128 && m >= 512 && !use_legacy &&
       aligned16(qw.words) && sb_aligned) {
-    const int cfg = pick_lds_cfg(m, n);
-    const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t192 = ((m + 191) / 192) * ((n + 255) / 256);
-    const bool tall = cfg == 0 || (cfg != 1 && (t256 + 255) / 256 * 256 <= (t192 + 255) / 256 * 192);
-    if (cfg != 2 || !getenv("KX355_GEMM_LDS_TILE")) {
-      if (tall) return launch_lds<256, 256, QB>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-      return launch_lds<192, 256, QB>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    const char* env = getenv("KX355_GEMM_LDS_TILE");
+    if (!env || env[0] != '2') {
+      if constexpr (QB != 0) {
+        if (quantized_tall(m, n)) launch_lds<256, QB>(a, lda, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+        else launch_lds<192, QB>(a, lda, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+      }
+      return KX_OK;
     }
   }
   switch (pick_cfg(m, n)) {
@@ -1832,16 +1285,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
   float v[4] = {acc.x, acc.y, acc.z, acc.w};
   epilogue_store4<H>(v, m, n, N, epi, C, ldc, vec_ok);
-}
-
-template <int BM, int BN, bool H>
-int launch_splitk(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, float* parts, int m, int n,
-                  int k, int splits, hipStream_t s) {
-  const dim3 grid((unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN)), (unsigned)splits);
-  const Epilogue plain{nullptr, nullptr, 0, nullptr, 1, 0, KX_EPI_OUT_F32};
-  gemm_lds_kernel<BM, BN, 0, false, 0, true, false, H><<<grid, 256, 0, s>>>(a, lda, w, ldw, QuantW{}, parts, n, m, n,
-                                                                   k / splits, plain);
-  return KX_OK;
 }
 
 // Tiled affine weights: for 256-row tile nb and 32-wide K stage kb, the rows' packed bytes of the
@@ -1985,6 +1428,8 @@ extern "C" int kx_gemm_qknorm_rope_bf16(const void* a, int64_t lda, const void* 
   epi.nq = norm_q;
   epi.nk = norm_k;
   epi.n_bf16 = norm_dtype == KX_BF16;
+  epi.head_dim = 128;
+  epi.sw_begin = n;
   epi.n_eps = eps;
   epi.n_off = weight_offset;
   epi.q_end = q_end;
@@ -2002,15 +1447,8 @@ extern "C" int kx_gemm_qknorm_rope_bf16(const void* a, int64_t lda, const void* 
   epi.t_shift = shift;
   epi.t_magic = (uint32_t)(((((unsigned __int128)1 << 32) * (uint64_t)((1ll << shift) - table_rows)) /
                             (uint64_t)table_rows) + 1);
-  const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t192 = ((m + 191) / 192) * ((n + 255) / 256);
-  const bool tall = (t256 + 255) / 256 * 256 <= (t192 + 255) / 256 * 192;
-  hipStream_t s = (hipStream_t)stream;
-  if (tall)
-    launch_lds_t<256, 256, 0, false, 0, false, true>((const uint16_t*)a, lda, (const uint16_t*)w, ldw, QuantW{}, c,
-                                                     ldc, (int)m, (int)n, (int)k, epi, s);
-  else
-    launch_lds_t<192, 256, 0, false, 0, false, true>((const uint16_t*)a, lda, (const uint16_t*)w, ldw, QuantW{}, c,
-                                                     ldc, (int)m, (int)n, (int)k, epi, s);
+  launch_dense_columns((const uint16_t*)a, lda, (const uint16_t*)w, ldw, c, ldc, (int)m, (int)n, (int)k, epi,
+                       (hipStream_t)stream);
   return check_launch(what);
 }
 
@@ -2166,16 +1604,14 @@ extern "C" int kx_qgemm_affine_tiled_bf16(const void* a, int64_t lda, const void
   if (m == 0) return KX_OK;
   const Epilogue epi{(const uint16_t*)bias, resid, ldr, gate, gate_div, gate_stride, epilogue};
   const QuantW qw{(const uint32_t*)wt, (const uint16_t*)sbt, nullptr};
-  const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t192 = ((m + 191) / 192) * ((n + 255) / 256);
-  const char* env = getenv("KX355_GEMM_LDS_TILE");
-  const bool tall = (env && *env) ? atoi(env) == 0 : (t256 + 255) / 256 * 256 <= (t192 + 255) / 256 * 192;
+  const bool tall = quantized_tall(m, n);
   hipStream_t s = (hipStream_t)stream;
   if (bits == 4) {
-    if (tall) launch_lds<256, 256, 4, true>((const uint16_t*)a, lda, nullptr, 0, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-    else launch_lds<192, 256, 4, true>((const uint16_t*)a, lda, nullptr, 0, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    if (tall) launch_lds<256, 4, true>((const uint16_t*)a, lda, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    else launch_lds<192, 4, true>((const uint16_t*)a, lda, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
   } else {
-    if (tall) launch_lds<256, 256, 8, true>((const uint16_t*)a, lda, nullptr, 0, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
-    else launch_lds<192, 256, 8, true>((const uint16_t*)a, lda, nullptr, 0, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    if (tall) launch_lds<256, 8, true>((const uint16_t*)a, lda, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    else launch_lds<192, 8, true>((const uint16_t*)a, lda, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
   }
   return check_launch("kx_qgemm_affine_tiled_bf16");
 }
@@ -2206,16 +1642,7 @@ int run_splitk(const char* what, const void* a, int64_t lda, const void* w, int6
                void* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int epilogue, const void* resid,
                int64_t ldr, const float* gate, int64_t gate_div, int64_t gate_stride, float* parts, int splits,
                hipStream_t s) {
-  // slices of 256x256 tiles for the tail rows of a large product (a few 256-row tiles across a wide
-  // N, each slice a quarter or less of K); up to 512 rows keep the 64x128 / 128x128 tiles
-  if (m > 512 && n >= 1024)
-    launch_splitk<256, 256, H>((const uint16_t*)a, lda, (const uint16_t*)w, ldw, parts, (int)m, (int)n, (int)k, splits,
-                            s);
-  else if (pick_lds_cfg(m, n) == 3)
-    launch_splitk<64, 128, H>((const uint16_t*)a, lda, (const uint16_t*)w, ldw, parts, (int)m, (int)n, (int)k, splits, s);
-  else
-    launch_splitk<128, 128, H>((const uint16_t*)a, lda, (const uint16_t*)w, ldw, parts, (int)m, (int)n, (int)k, splits,
-                            s);
+  launch_dense_slices(H, (const uint16_t*)a, lda, (const uint16_t*)w, ldw, parts, (int)m, (int)n, (int)k, splits, s);
   const Epilogue epi{(const uint16_t*)bias, resid, ldr, gate, gate_div, gate_stride, epilogue};
   const bool vec_ok = (ldc % 4 == 0) && (!(epilogue & KX_EPI_GATED_RESIDUAL) || ldr % 4 == 0);
   const int64_t threads = m * (n / 4);
@@ -2288,6 +1715,14 @@ int splitk_entry(const void* a, int64_t lda, const void* w, int64_t ldw, const v
 
 KX_SPLITK_ENTRY(bf16, false)
 KX_SPLITK_ENTRY(f16, true)
+
+extern "C" int kx_gemm_splits(int64_t m, int64_t n, int64_t k, int* splits) {
+  KX_REQUIRE(splits, "kx_gemm_splits: null result");
+  KX_REQUIRE(m >= 0 && n >= 0 && k > 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 30),
+             "kx_gemm_splits: bad shape (%lld, %lld, %lld)", (long long)m, (long long)n, (long long)k);
+  *splits = m == 0 || n == 0 || n % 4 || k % DENSE_BK ? 1 : dense_splits(m, n, k);
+  return KX_OK;
+}
 
 extern "C" int kx_gemm_splitk_noalloc_bf16(const void* a, int64_t lda, const void* w, int64_t ldw,
                                            const void* bias, void* c, int64_t ldc, int64_t m, int64_t n, int64_t k,
