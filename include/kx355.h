@@ -267,6 +267,23 @@ int kx_gemm_qknorm_rope_bf16(const void* a, int64_t lda, const void* w, int64_t 
                              int64_t table_rows, int64_t table_bs, kx_stream_t stream);
 
 /*
+ * The general form: query and key heads of head_dim (64 or 128) columns as above (none when
+ * k_end == 0: the norm weights and tables may then be null), and the columns from swiglu_begin on a
+ * SwiGLU pair: F = (n - swiglu_begin) / 2 gate columns, then F up columns, leave as
+ * c2[m, f] = silu(gate) * up (bf16, row stride ldc2), both formed and multiplied in fp32; c takes the
+ * columns before swiglu_begin only (null when there are none). swiglu_begin == n: no SwiGLU columns
+ * (c2 null). swiglu_begin and 2 F are multiples of 256, q_end and k_end of 128. Replaces linear_in +
+ * swiglu of the FLUX.2 feed-forward and single block (kinomlx/models/flux2/transformer.py:63-85,
+ * 170-198) and gate / up of Krea2SwiGLU (kinomlx/models/krea2/transformer/model.py:199-214).
+ */
+int kx_gemm_columns_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias, void* c,
+                         int64_t ldc, int64_t m, int64_t n, int64_t k, int64_t q_end, int64_t k_end,
+                         int64_t head_dim, const void* norm_q, const void* norm_k, int norm_dtype, float eps,
+                         float weight_offset, const float* cos, const float* sin, int64_t table_ld,
+                         int64_t table_hs, int64_t table_rows, int64_t table_bs, int64_t swiglu_begin, void* c2,
+                         int64_t ldc2, kx_stream_t stream);
+
+/*
  * Group-wise affine int4/int8 weight-quantized linear, dequantized inside the MFMA mainloop:
  * replaces nn.QuantizedLinear / mx.quantized_matmul(x, wq, scales, biases, transpose=True,
  * group_size, bits, mode="affine") + bias (kinomlx/models/ltx2/weights/quantization.py:28-44,

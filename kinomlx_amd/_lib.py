@@ -101,6 +101,10 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I, _F, _F, _P, _P, _I64, _I64,
         _I64, _I64, _P,
     ],
+    "kx_gemm_columns_bf16": [
+        _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I, _F, _F, _P, _P, _I64, _I64,
+        _I64, _I64, _I64, _P, _I64, _P,
+    ],
     "kx_qgemm_mxfp8_bf16": [
         _P, _I64, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P, _I64, _I64, _P,
     ],
@@ -526,6 +530,49 @@ def launch_gemm_qknorm_rope(a, w, out, *, bias, q_end: int, k_end: int, norm_q, 
         "kx_gemm_qknorm_rope_bf16", _ptr(a), lda, _ptr(w), ldw, _ptr(bias), _ptr(out), ldc, m, n, k, q_end, k_end,
         _ptr(norm_q), _ptr(norm_k), KX_BF16 if norm_q.dtype == torch.bfloat16 else KX_F32, float(eps),
         float(weight_offset), _ptr(cos), _ptr(sin), table_ld, table_hs, table_rows, table_bs, _stream(),
+    )
+
+
+def launch_gemm_columns(a, w, out, *, bias=None, q_end: int = 0, k_end: int = 0, head_dim: int = 128, norm_q=None,
+                        norm_k=None, eps: float = 0.0, weight_offset: float = 0.0, cos=None, sin=None,
+                        table_ld: int = 0, table_hs: int = 0, table_rows: int = 1, table_bs: int = 0,
+                        swiglu_begin: int | None = None, swiglu_out=None) -> None:
+    """``a @ w.T + bias`` with its column forms: query / key heads of ``head_dim`` normalized and rotated
+    as in ``launch_gemm_qknorm_rope`` (``k_end`` 0: none), and the columns from ``swiglu_begin`` on,
+    ``[gate | up]``, written as ``silu(gate) * up`` to ``swiglu_out`` (None: no such columns). ``out``
+    holds the columns before ``swiglu_begin`` (None when there are none)."""
+    _check_gpu("gemm_columns", a, w, out, bias, norm_q, norm_k, cos, sin, swiglu_out)
+    m, k, lda = _rows(a, "projection input")
+    n, kw, ldw = _rows(w, "projection weight")
+    _same_dtype("gemm_columns", torch.bfloat16, a, w, bias, out, swiglu_out)
+    if kw != k:
+        raise ValueError(f"projection: input width {k} does not match weight width {kw}")
+    begin = n if swiglu_out is None else swiglu_begin
+    ldc = ldc2 = 0
+    if out is not None:
+        rows, nout, ldc = _rows(out, "projection output")
+        if rows != m or nout != begin:
+            raise ValueError(f"projection: out must hold {m} rows of {begin} columns")
+    elif begin:
+        raise ValueError("projection: no output for its plain columns")
+    if swiglu_out is not None:
+        rows, nout, ldc2 = _rows(swiglu_out, "SwiGLU output")
+        if rows != m or 2 * nout != n - begin:
+            raise ValueError(f"projection: the SwiGLU output must hold {m} rows of {(n - begin) // 2} columns")
+    code = KX_F32
+    if k_end:
+        if norm_q.dtype != norm_k.dtype or norm_q.dtype not in (torch.float32, torch.bfloat16):
+            raise ValueError("projection: norm weights must both be fp32 or both bf16")
+        if norm_q.shape != (head_dim,) or norm_k.shape != (head_dim,) \
+                or not (norm_q.is_contiguous() and norm_k.is_contiguous()):
+            raise ValueError(f"projection: norm weights must be contiguous ({head_dim},)")
+        if cos.dtype != torch.float32 or sin.dtype != torch.float32:
+            raise ValueError("projection: rotary tables must be fp32")
+        code = KX_BF16 if norm_q.dtype == torch.bfloat16 else KX_F32
+    _call(
+        "kx_gemm_columns_bf16", _ptr(a), lda, _ptr(w), ldw, _ptr(bias), _ptr(out), ldc, m, n, k, q_end, k_end, head_dim,
+        _ptr(norm_q), _ptr(norm_k), code, float(eps), float(weight_offset), _ptr(cos), _ptr(sin), table_ld, table_hs,
+        table_rows, table_bs, begin, _ptr(swiglu_out), ldc2, _stream(),
     )
 
 

@@ -6,8 +6,8 @@
 // (out, in) weight layout), fp32 accumulation, one rounding to the 16-bit type (bf16, or fp16 for
 // dense operands, template H).
 //
-// The register-staged kernel (v_mfma_f32_32x32x16): a BM x BN output tile per workgroup of WM x WN waves; each wave owns a
-// (BM/WM) x (BN/WN) sub-tile as a grid of 32x32 MFMA blocks. K advances in stages of 64: the
+// The register-staged kernel (v_mfma_f32_32x32x16): a BM x BN output tile per workgroup of WM x WN
+// waves; each wave owns a (BM/WM) x (BN/WN) sub-tile as a grid of 32x32 MFMA blocks. K advances in stages of 64: the
 // next stage's global loads are issued into registers before the current stage's MFMAs and
 // written to the other half of a double-buffered LDS tile afterwards, so one barrier per stage
 // suffices. LDS rows are 128 bytes (64 bf16) with the 16-byte chunk index XOR-swizzled by the
@@ -1391,6 +1391,83 @@ extern "C" int kx_gemm_f16(const void* a, int64_t lda, const void* w, int64_t ld
                           (hipStream_t)stream);
 }
 
+namespace {
+// The column forms' shared entry: query / key heads of head_dim columns normalized and rotated, the
+// columns from swiglu_begin on a SwiGLU pair written to c2.
+int gemm_columns(const char* what, const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias, void* c,
+                 int64_t ldc, int64_t m, int64_t n, int64_t k, int64_t q_end, int64_t k_end, int64_t head_dim,
+                 const void* norm_q, const void* norm_k, int norm_dtype, float eps, float weight_offset,
+                 const float* cos, const float* sin, int64_t table_ld, int64_t table_hs, int64_t table_rows,
+                 int64_t table_bs, int64_t swiglu_begin, void* c2, int64_t ldc2, hipStream_t s) {
+  KX_REQUIRE(a && w && (c || swiglu_begin == 0) && (c2 || swiglu_begin == n), "%s: null tensor", what);
+  KX_REQUIRE(k_end == 0 || (norm_q && norm_k && cos && sin), "%s: null tensor", what);
+  KX_REQUIRE(m >= 0 && n > 0 && k > 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 30) &&
+                 k % DENSE_BK == 0,
+             "%s: bad shape (m=%lld n=%lld k=%lld; k %% 64 == 0)", what, (long long)m, (long long)n, (long long)k);
+  KX_REQUIRE(head_dim == 64 || head_dim == 128, "%s: head_dim must be 64 or 128, got %lld", what, (long long)head_dim);
+  KX_REQUIRE(q_end >= 0 && q_end % 128 == 0 && k_end >= q_end && k_end % 128 == 0 && k_end <= swiglu_begin,
+             "%s: the query and key columns must be whole 128-wide heads inside n (q_end=%lld k_end=%lld)", what,
+             (long long)q_end, (long long)k_end);
+  KX_REQUIRE(swiglu_begin >= 0 && swiglu_begin <= n &&
+                 (swiglu_begin == n || (swiglu_begin % 256 == 0 && (n - swiglu_begin) % 256 == 0)),
+             "%s: the SwiGLU columns must start at a multiple of 256 and be a multiple of 256 (begin=%lld n=%lld)",
+             what, (long long)swiglu_begin, (long long)n);
+  KX_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= k && ldw >= k && lda <= (1 << 22) && ldw <= (1 << 22) &&
+                 (swiglu_begin == 0 || (ldc >= swiglu_begin && ldc % 4 == 0)) &&
+                 (swiglu_begin == n || (ldc2 >= (n - swiglu_begin) / 2 && ldc2 % 4 == 0)),
+             "%s: bad strides", what);
+  // a SwiGLU tile addresses its up rows from its gate rows with a 32-bit byte offset
+  KX_REQUIRE(swiglu_begin == n || ((n - swiglu_begin) / 2 + 256) * ldw * 2 < (1ll << 32),
+             "%s: SwiGLU weight rows are too far apart", what);
+  KX_REQUIRE(aligned16(a) && aligned16(w) && aligned8(c) && aligned8(c2) && (!bias || aligned8(bias)),
+             "%s: misaligned tensor", what);
+  Epilogue epi{(const uint16_t*)bias, nullptr, 0, nullptr, 1, 0, bias ? KX_EPI_BIAS : 0};
+  epi.sw_begin = swiglu_begin;
+  epi.sw_width = (n - swiglu_begin) / 2;
+  epi.c2 = c2;
+  epi.ldc2 = ldc2;
+  if (k_end > 0) {
+    KX_REQUIRE(norm_dtype == KX_F32 || norm_dtype == KX_BF16, "%s: norm weights must be KX_F32 or KX_BF16", what);
+    KX_REQUIRE(norm_dtype == KX_BF16 ? (aligned8(norm_q) && aligned8(norm_k))
+                                     : (aligned16(norm_q) && aligned16(norm_k)),
+               "%s: misaligned norm weights", what);
+    KX_REQUIRE(aligned16(cos) && aligned16(sin) && table_ld % 4 == 0 && table_hs % 4 == 0 && table_bs % 4 == 0 &&
+                   table_rows > 0 && table_rows < (1ll << 31),
+               "%s: tables need 16-byte aligned rows (table_ld, table_hs, table_bs multiples of 4)", what);
+    // the kernel indexes the tables with 32-bit offsets
+    const int64_t heads = std::max(q_end, k_end - q_end) / head_dim;
+    const int64_t last = (m > 0 ? (m - 1) / table_rows : 0) * table_bs + std::min(m, table_rows) * table_ld +
+                         std::max<int64_t>(heads - 1, 0) * table_hs + head_dim;
+    KX_REQUIRE(table_ld >= 0 && table_hs >= 0 && table_bs >= 0 && last < (1ll << 31),
+               "%s: table offsets must be non-negative and below 2^31 elements", what);
+    epi.nq = norm_q;
+    epi.nk = norm_k;
+    epi.n_bf16 = norm_dtype == KX_BF16;
+    epi.head_dim = (int)head_dim;
+    epi.n_eps = eps;
+    epi.n_off = weight_offset;
+    epi.q_end = q_end;
+    epi.k_end = k_end;
+    epi.cosp = cos;
+    epi.sinp = sin;
+    epi.t_ld = table_ld;
+    epi.t_hs = table_hs;
+    epi.t_rows = table_rows;
+    epi.t_bs = table_bs;
+    // division by the invariant table_rows (round-up method): shift = ceil(log2 d),
+    // magic = floor(2^32 (2^shift - d) / d) + 1
+    int shift = 0;
+    while ((1ll << shift) < table_rows) ++shift;
+    epi.t_shift = shift;
+    epi.t_magic = (uint32_t)(((((unsigned __int128)1 << 32) * (uint64_t)((1ll << shift) - table_rows)) /
+                              (uint64_t)table_rows) + 1);
+  }
+  if (m == 0) return KX_OK;
+  launch_dense_columns((const uint16_t*)a, lda, (const uint16_t*)w, ldw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+  return check_launch(what);
+}
+}  // namespace
+
 extern "C" int kx_gemm_qknorm_rope_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias,
                                         void* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int64_t q_end,
                                         int64_t k_end, const void* norm_q, const void* norm_k, int norm_dtype,
@@ -1398,58 +1475,21 @@ extern "C" int kx_gemm_qknorm_rope_bf16(const void* a, int64_t lda, const void* 
                                         int64_t table_ld, int64_t table_hs, int64_t table_rows, int64_t table_bs,
                                         kx_stream_t stream) {
   const char* what = "kx_gemm_qknorm_rope_bf16";
-  KX_REQUIRE(a && w && c && norm_q && norm_k && cos && sin, "%s: null tensor", what);
-  KX_REQUIRE(m >= 0 && n > 0 && k > 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 30) &&
-                 k % DENSE_BK == 0,
-             "%s: bad shape (m=%lld n=%lld k=%lld; k %% 64 == 0)", what, (long long)m, (long long)n, (long long)k);
-  KX_REQUIRE(q_end >= 0 && q_end % 128 == 0 && k_end >= q_end && k_end % 128 == 0 && k_end <= n,
-             "%s: the query and key columns must be whole 128-wide heads inside n (q_end=%lld k_end=%lld)", what,
-             (long long)q_end, (long long)k_end);
-  KX_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= k && ldw >= k && ldc >= n && ldc % 4 == 0 && lda <= (1 << 22) &&
-                 ldw <= (1 << 22),
-             "%s: bad strides", what);
-  KX_REQUIRE(aligned16(a) && aligned16(w) && aligned8(c) && (!bias || aligned8(bias)), "%s: misaligned tensor", what);
-  KX_REQUIRE(norm_dtype == KX_F32 || norm_dtype == KX_BF16, "%s: norm weights must be KX_F32 or KX_BF16", what);
-  KX_REQUIRE(norm_dtype == KX_BF16 ? (aligned8(norm_q) && aligned8(norm_k)) : (aligned16(norm_q) && aligned16(norm_k)),
-             "%s: misaligned norm weights", what);
-  KX_REQUIRE(aligned16(cos) && aligned16(sin) && table_ld % 4 == 0 && table_hs % 4 == 0 && table_bs % 4 == 0 &&
-                 table_rows > 0 && table_rows < (1ll << 31),
-             "%s: tables need 16-byte aligned rows (table_ld, table_hs, table_bs multiples of 4)", what);
-  {
-    // the kernel indexes the tables with 32-bit offsets
-    const int64_t heads = std::max(q_end, k_end - q_end) / 128;
-    const int64_t last = (m > 0 ? (m - 1) / table_rows : 0) * table_bs + std::min(m, table_rows) * table_ld +
-                         std::max<int64_t>(heads - 1, 0) * table_hs + 128;
-    KX_REQUIRE(table_ld >= 0 && table_hs >= 0 && table_bs >= 0 && last < (1ll << 31),
-               "%s: table offsets must be non-negative and below 2^31 elements", what);
-  }
-  if (m == 0) return KX_OK;
-  Epilogue epi{(const uint16_t*)bias, nullptr, 0, nullptr, 1, 0, bias ? KX_EPI_BIAS : 0};
-  epi.nq = norm_q;
-  epi.nk = norm_k;
-  epi.n_bf16 = norm_dtype == KX_BF16;
-  epi.head_dim = 128;
-  epi.sw_begin = n;
-  epi.n_eps = eps;
-  epi.n_off = weight_offset;
-  epi.q_end = q_end;
-  epi.k_end = k_end;
-  epi.cosp = cos;
-  epi.sinp = sin;
-  epi.t_ld = table_ld;
-  epi.t_hs = table_hs;
-  epi.t_rows = table_rows;
-  epi.t_bs = table_bs;
-  // division by the invariant table_rows (round-up method): shift = ceil(log2 d),
-  // magic = floor(2^32 (2^shift - d) / d) + 1
-  int shift = 0;
-  while ((1ll << shift) < table_rows) ++shift;
-  epi.t_shift = shift;
-  epi.t_magic = (uint32_t)(((((unsigned __int128)1 << 32) * (uint64_t)((1ll << shift) - table_rows)) /
-                            (uint64_t)table_rows) + 1);
-  launch_dense_columns((const uint16_t*)a, lda, (const uint16_t*)w, ldw, c, ldc, (int)m, (int)n, (int)k, epi,
-                       (hipStream_t)stream);
-  return check_launch(what);
+  KX_REQUIRE(c && norm_q && norm_k && cos && sin, "%s: null tensor", what);
+  return gemm_columns(what, a, lda, w, ldw, bias, c, ldc, m, n, k, q_end, k_end, 128, norm_q, norm_k, norm_dtype, eps,
+                      weight_offset, cos, sin, table_ld, table_hs, table_rows, table_bs, n, nullptr, 0,
+                      (hipStream_t)stream);
+}
+
+extern "C" int kx_gemm_columns_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias, void* c,
+                                    int64_t ldc, int64_t m, int64_t n, int64_t k, int64_t q_end, int64_t k_end,
+                                    int64_t head_dim, const void* norm_q, const void* norm_k, int norm_dtype,
+                                    float eps, float weight_offset, const float* cos, const float* sin,
+                                    int64_t table_ld, int64_t table_hs, int64_t table_rows, int64_t table_bs,
+                                    int64_t swiglu_begin, void* c2, int64_t ldc2, kx_stream_t stream) {
+  return gemm_columns("kx_gemm_columns_bf16", a, lda, w, ldw, bias, c, ldc, m, n, k, q_end, k_end, head_dim, norm_q,
+                      norm_k, norm_dtype, eps, weight_offset, cos, sin, table_ld, table_hs, table_rows, table_bs,
+                      swiglu_begin, c2, ldc2, (hipStream_t)stream);
 }
 
 extern "C" int kx_qgemm_affine_bf16(const void* a, int64_t lda, const uint32_t* wq,

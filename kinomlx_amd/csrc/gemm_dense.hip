@@ -225,6 +225,25 @@ __device__ __forceinline__ void strip_norm_rope(const float* st, int rr, int c4,
   }
 }
 
+// silu(gate) * up of 4 columns of a row staged at g and u.
+__device__ __forceinline__ uint2 swiglu4(const float* g, const float* u, const float* bg, const float* bu) {
+  const float4 a = *reinterpret_cast<const float4*>(g), b = *reinterpret_cast<const float4*>(u);
+  uint2 o;
+  o.x = pack2(fast_silu(a.x + bg[0]) * (b.x + bu[0]), fast_silu(a.y + bg[1]) * (b.y + bu[1]));
+  o.y = pack2(fast_silu(a.z + bg[2]) * (b.z + bu[2]), fast_silu(a.w + bg[3]) * (b.w + bu[3]));
+  return o;
+}
+__device__ __forceinline__ void swiglu_bias(const Epilogue& epi, int ng, int nu, float* bg, float* bu) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) bg[e] = bu[e] = 0.0f;
+  if (epi.flags & KX_EPI_BIAS) {
+    const uint2 x = *reinterpret_cast<const uint2*>(epi.bias + ng);
+    const uint2 y = *reinterpret_cast<const uint2*>(epi.bias + nu);
+    bg[0] = lo_f(x.x); bg[1] = hi_f(x.x); bg[2] = lo_f(x.y); bg[3] = hi_f(x.y);
+    bu[0] = lo_f(y.x); bu[1] = hi_f(y.x); bu[2] = lo_f(y.y); bu[3] = hi_f(y.y);
+  }
+}
+
 // ---- 256 x 256 and 128 x 256 tiles ---------------------------------------------------------------
 //
 // Waves 2 (rows) x 4 (columns); the tile's rows and columns are two halves each, and a wave owns
@@ -416,13 +435,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(const uint16_t* __restr
   if constexpr (NS) {
     if (swiglu) {
       uint16_t* out = static_cast<uint16_t*>(epi.c2) + (n0 - (int)epi.sw_begin) + c4;
-      float bg[4] = {0.0f, 0.0f, 0.0f, 0.0f}, bu[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (epi.flags & KX_EPI_BIAS) {
-        const uint2 x = *reinterpret_cast<const uint2*>(epi.bias + n0 + c4);
-        const uint2 y = *reinterpret_cast<const uint2*>(epi.bias + n0 + whalf + c4);
-        bg[0] = lo_f(x.x); bg[1] = hi_f(x.x); bg[2] = lo_f(x.y); bg[3] = hi_f(x.y);
-        bu[0] = lo_f(y.x); bu[1] = hi_f(y.x); bu[2] = lo_f(y.y); bu[3] = hi_f(y.y);
-      }
+      float bg[4], bu[4];
+      swiglu_bias(epi, n0 + c4, n0 + whalf + c4, bg, bu);
 #pragma unroll
       for (int ha = 0; ha < 2; ++ha) {
         if (ha) KX_BARRIER();  // the first half's strips have been read
@@ -433,11 +447,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(const uint16_t* __restr
 #pragma unroll
         for (int q = 0; q < NROW; ++q) {
           const int r = rr + q * STEP, m = m0 + ha * HA + r;
-          const float4 g = *reinterpret_cast<const float4*>(strip + r * PITCH + c4);
-          const float4 u = *reinterpret_cast<const float4*>(strip + STRIP + r * PITCH + c4);
-          uint2 o;
-          o.x = pack2(fast_silu(g.x + bg[0]) * (u.x + bu[0]), fast_silu(g.y + bg[1]) * (u.y + bu[1]));
-          o.y = pack2(fast_silu(g.z + bg[2]) * (u.z + bu[2]), fast_silu(g.w + bg[3]) * (u.w + bu[3]));
+          const uint2 o = swiglu4(strip + r * PITCH + c4, strip + STRIP + r * PITCH + c4, bg, bu);
           if (m < M) *reinterpret_cast<uint2*>(out + (int64_t)m * epi.ldc2) = o;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -477,7 +487,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(const uint16_t* __restr
 // waves (2 x 2), a ring of four 64-wide stages with the copies three stages ahead between the MFMAs;
 // every k32 step waits for its fragments (read one step earlier), then each MFMA is followed by its
 // share of the next step's reads and of the copies. The last step of a stage holds its only barrier.
-template <int BM, int GMODE, bool OUTF32, bool H>
+// NS: the column forms, as in gemm_pp_kernel; a SwiGLU tile pairs 64 gate with 64 up columns.
+template <int BM, int GMODE, bool OUTF32, bool NS, bool H>
 __global__ __launch_bounds__(256) void gemm_ring_kernel(const uint16_t* __restrict__ A, int64_t lda,
                                                         const uint16_t* __restrict__ W, int64_t ldw,
                                                         void* __restrict__ C, int64_t ldc, int M, int N, int K,
@@ -504,10 +515,18 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const uint16_t* __restri
     W += y * K;
     C = static_cast<float*>(C) + y * (int64_t)M * ldc;
   }
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int tiles_m = (M + BM - 1) / BM;
+  int plain_n = (N + BN - 1) / BN, tiles_n = plain_n;
+  if constexpr (NS) {
+    plain_n = ((int)epi.sw_begin + BN - 1) / BN;
+    tiles_n = plain_n + (int)(epi.sw_width / 64);
+  }
   int2 tile = lds_tile_of(blockIdx.x, tiles_m, tiles_n);
   if (epi.rows_desc) tile.x = tiles_m - 1 - tile.x;
-  const int m0 = tile.x * BM, n0 = tile.y * BN;
+  const int m0 = tile.x * BM;
+  const bool swiglu = NS && tile.y >= plain_n;
+  const int n0 = swiglu ? (int)epi.sw_begin + (tile.y - plain_n) * 64 : tile.y * BN;
+  const int wskip = swiglu ? (int)epi.sw_width - 64 : 0;  // weight rows between the tile's two halves
   const i32x4 abuf = buffer_of(A + (int64_t)m0 * lda), wbuf = buffer_of(W + (int64_t)n0 * ldw);
   const int r8 = lane >> 3, slot = lane & 7;
   uint32_t vo[PER];
@@ -519,7 +538,8 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const uint16_t* __restri
 #pragma unroll
   for (int i = 0; i < W_INST; ++i) {
     const int r = (wave * W_INST + i) * 8 + r8;
-    vo[A_INST + i] = (uint32_t)(((int64_t)(min(n0 + r, N - 1) - n0) * ldw + (slot ^ ((r >> 1) & 7)) * 8) * 2);
+    const int wr = r + (r < 64 ? 0 : wskip);
+    vo[A_INST + i] = (uint32_t)(((int64_t)(min(n0 + wr, N - 1) - n0) * ldw + (slot ^ ((r >> 1) & 7)) * 8) * 2);
   }
   const uint32_t lds0 = lds_address(smem);
   auto copy = [&](int i, int buf, uint32_t ko) {
@@ -608,7 +628,27 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const uint16_t* __restri
           make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   KX_BARRIER();
-  strip_store<H, GMODE, OUTF32, NROW, STEP>(strip, rr, c4, m0, n0 + c4, M, N, epi, full, vec_ok, res, C, ldc);
+  if constexpr (NS) {
+    if (swiglu) {
+      const int p4 = (tid & 15) * 4;
+      float bg[4], bu[4];
+      swiglu_bias(epi, n0 + p4, n0 + (int)epi.sw_width + p4, bg, bu);
+      uint16_t* out = static_cast<uint16_t*>(epi.c2) + (n0 - (int)epi.sw_begin) + p4;
+#pragma unroll
+      for (int q = 0; q < BM / 16; ++q) {
+        const int r = (tid >> 4) + q * 16, m = m0 + r;
+        const uint2 o = swiglu4(strip + r * PITCH + p4, strip + r * PITCH + 64 + p4, bg, bu);
+        if (m < M) *reinterpret_cast<uint2*>(out + (int64_t)m * epi.ldc2) = o;
+      }
+      return;
+    }
+    if (n0 < epi.k_end) {
+      strip_norm_rope<NROW, STEP>(strip, rr, c4, m0, n0 + c4, M, epi, static_cast<uint16_t*>(C), ldc);
+      return;
+    }
+  }
+  strip_store<H, GMODE, OUTF32, NROW, STEP>(strip, rr, c4, m0, n0 + c4, M, NS ? min(N, (int)epi.sw_begin) : N, epi,
+                                            full, vec_ok, res, C, ldc);
 }
 
 // ---- launches ------------------------------------------------------------------------------------
@@ -629,21 +669,25 @@ void run_pp(const Call& x, const Epilogue& epi, int tiles_n) {
   const dim3 grid((unsigned)(((x.m + BM - 1) / BM) * tiles_n), (unsigned)x.splits);
   gemm_pp_kernel<BM, GMODE, OUTF32, NS, H><<<grid, 512, 0, x.s>>>(x.a, x.lda, x.w, x.ldw, x.c, x.ldc, x.m, x.n, x.k, epi);
 }
-template <int BM, int GMODE, bool OUTF32, bool H>
-void run_ring(const Call& x, const Epilogue& epi) {
-  const dim3 grid((unsigned)(((x.m + BM - 1) / BM) * ((x.n + 127) / 128)), (unsigned)x.splits);
-  gemm_ring_kernel<BM, GMODE, OUTF32, H><<<grid, 256, 0, x.s>>>(x.a, x.lda, x.w, x.ldw, x.c, x.ldc, x.m, x.n, x.k, epi);
+template <int BM, int GMODE, bool OUTF32, bool NS, bool H>
+void run_ring(const Call& x, const Epilogue& epi, int tiles_n) {
+  const dim3 grid((unsigned)(((x.m + BM - 1) / BM) * tiles_n), (unsigned)x.splits);
+  gemm_ring_kernel<BM, GMODE, OUTF32, NS, H><<<grid, 256, 0, x.s>>>(x.a, x.lda, x.w, x.ldw, x.c, x.ldc, x.m, x.n, x.k, epi);
 }
 
-template <int GMODE, bool OUTF32, bool H>
-void run_tile(int tile, const Call& x, const Epilogue& epi) {
-  const int tiles_n = (x.n + 255) / 256;
+// tiles_256, tiles_128: the product's column tiles of either width
+template <int GMODE, bool OUTF32, bool NS, bool H>
+void run_tile(int tile, const Call& x, const Epilogue& epi, int tiles_256, int tiles_128) {
   switch (tile) {
-    case DT256x256: return run_pp<256, GMODE, OUTF32, false, H>(x, epi, tiles_n);
-    case DT128x256: return run_pp<128, GMODE, OUTF32, false, H>(x, epi, tiles_n);
-    case DT128x128: return run_ring<128, GMODE, OUTF32, H>(x, epi);
-    default: return run_ring<64, GMODE, OUTF32, H>(x, epi);
+    case DT256x256: return run_pp<256, GMODE, OUTF32, NS, H>(x, epi, tiles_256);
+    case DT128x256: return run_pp<128, GMODE, OUTF32, NS, H>(x, epi, tiles_256);
+    case DT128x128: return run_ring<128, GMODE, OUTF32, NS, H>(x, epi, tiles_128);
+    default: return run_ring<64, GMODE, OUTF32, NS, H>(x, epi, tiles_128);
   }
+}
+template <int GMODE, bool OUTF32, bool H>
+void run_plain(int tile, const Call& x, const Epilogue& epi) {
+  run_tile<GMODE, OUTF32, false, H>(tile, x, epi, (x.n + 255) / 256, (x.n + 127) / 128);
 }
 
 // Residual mode (none / 16-bit / fp32) and output type select the epilogue.
@@ -652,12 +696,12 @@ void run_epilogue(int tile, const Call& x, const Epilogue& epi) {
   const int gmode = (epi.flags & KX_EPI_GATED_RESIDUAL) ? ((epi.flags & KX_EPI_RESID_F32) ? 2 : 1) : 0;
   const bool out32 = epi.flags & KX_EPI_OUT_F32;
   switch (gmode * 2 + (out32 ? 1 : 0)) {
-    case 0: return run_tile<0, false, H>(tile, x, epi);
-    case 1: return run_tile<0, true, H>(tile, x, epi);
-    case 2: return run_tile<1, false, H>(tile, x, epi);
-    case 3: return run_tile<1, true, H>(tile, x, epi);
-    case 4: return run_tile<2, false, H>(tile, x, epi);
-    default: return run_tile<2, true, H>(tile, x, epi);
+    case 0: return run_plain<0, false, H>(tile, x, epi);
+    case 1: return run_plain<0, true, H>(tile, x, epi);
+    case 2: return run_plain<1, false, H>(tile, x, epi);
+    case 3: return run_plain<1, true, H>(tile, x, epi);
+    case 4: return run_plain<2, false, H>(tile, x, epi);
+    default: return run_plain<2, true, H>(tile, x, epi);
   }
 }
 
@@ -702,10 +746,10 @@ double tile_cost(const TileCost& t, int64_t m, int64_t n, int64_t k, int64_t sli
          (rest > 0 ? stages * (t.part + t.load * (double)rest / (double)kCUs) : 0.0);
 }
 
-// The fastest tile of the first `count` sizes.
-int best_tile(int64_t m, int64_t n, int64_t k, int count, double* cost) {
+// The fastest tile size.
+int best_tile(int64_t m, int64_t n, int64_t k, double* cost) {
   int best = 0;
-  for (int i = 0; i < count; ++i) {
+  for (int i = 0; i < 4; ++i) {
     const double c = tile_cost(kTiles[i], m, n, k);
     if (i == 0 || c < *cost) {
       best = i;
@@ -723,9 +767,9 @@ struct RowPlan {
   int64_t rows;
   int tile, rest_tile;
 };
-RowPlan row_plan(int64_t m, int64_t n, int64_t k, int count) {
+RowPlan row_plan(int64_t m, int64_t n, int64_t k) {
   double cost = 0.0;
-  RowPlan plan{0, best_tile(m, n, k, count, &cost), 0};
+  RowPlan plan{0, best_tile(m, n, k, &cost), 0};
   const int64_t tiles_n = (n + 255) / 256, tiles_m = (m + 255) / 256;
   // a split has to win 4 %, the error of the rule
   double limit = 0.96 * cost;
@@ -734,7 +778,7 @@ RowPlan row_plan(int64_t m, int64_t n, int64_t k, int count) {
     const int64_t rows = r * kCUs / tiles_n * 256;
     if (rows == 0 || rows >= m) continue;
     double rest = 0.0;
-    const int rest_tile = best_tile(m - rows, n, k, count, &rest);
+    const int rest_tile = best_tile(m - rows, n, k, &rest);
     const double c = tile_cost(kTiles[0], rows, n, k) + rest;
     if (c < limit) {
       limit = c;
@@ -754,9 +798,9 @@ int forced_tile() {
 // Call `run(first row, rows, tile)` for each part of the plan; the last rows first (their producer
 // wrote them most recently, and their pass leaves the weight in the memory-side cache).
 template <typename F>
-void run_rows(int64_t m, int64_t n, int64_t k, int count, F run) {
+void run_rows(int64_t m, int64_t n, int64_t k, F run) {
   const int forced = forced_tile();
-  const RowPlan p = forced >= 0 ? RowPlan{0, std::min(forced, count - 1), 0} : row_plan(m, n, k, count);
+  const RowPlan p = forced >= 0 ? RowPlan{0, forced, 0} : row_plan(m, n, k);
   if (p.rows) run(p.rows, m - p.rows, p.rest_tile);
   run(0, p.rows ? p.rows : m, p.tile);
 }
@@ -781,9 +825,9 @@ int slice_tile(int64_t m, int64_t n, int64_t k, int s, double* cost) {
 int dense_splits(int64_t m, int64_t n, int64_t k) {
   // a row plan's parts cost the sum of theirs
   double cost = 0.0;
-  const RowPlan p = row_plan(m, n, k, 4);
+  const RowPlan p = row_plan(m, n, k);
   if (p.rows) {
-    best_tile(m - p.rows, n, k, 4, &cost);
+    best_tile(m - p.rows, n, k, &cost);
     cost += tile_cost(kTiles[0], p.rows, n, k);
   } else {
     cost = tile_cost(kTiles[p.tile], m, n, k);
@@ -804,7 +848,7 @@ int dense_splits(int64_t m, int64_t n, int64_t k) {
 
 void launch_dense(bool half, const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, void* c, int64_t ldc,
                   int m, int n, int k, const Epilogue& epi, hipStream_t s) {
-  run_rows(m, n, k, 4, [&](int64_t row0, int64_t rows, int tile) {
+  run_rows(m, n, k, [&](int64_t row0, int64_t rows, int tile) {
     Epilogue e = epi;
     e.rows_desc = rows_last_first(rows, k);
     e.row0 = row0;
@@ -826,21 +870,21 @@ void launch_dense_slices(bool half, const uint16_t* a, int64_t lda, const uint16
   double cost = 0.0;
   const int tile = forced >= 0 ? forced : slice_tile(m, n, k, splits, &cost);
   const Call x{a, lda, w, ldw, parts, n, m, n, k / splits, splits, s};
-  if (half) run_tile<0, true, true>(tile, x, plain);
-  else run_tile<0, true, false>(tile, x, plain);
+  if (half) run_plain<0, true, true>(tile, x, plain);
+  else run_plain<0, true, false>(tile, x, plain);
 }
 
 void launch_dense_columns(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, void* c, int64_t ldc, int m,
                           int n, int k, const Epilogue& epi, hipStream_t s) {
-  const int tiles_n = (int)((epi.sw_begin + 255) / 256 + epi.sw_width / 128);
-  run_rows(m, (int64_t)tiles_n * 256, k, 2, [&](int64_t row0, int64_t rows, int tile) {
+  const int t256 = (int)((epi.sw_begin + 255) / 256 + epi.sw_width / 128);
+  const int t128 = (int)((epi.sw_begin + 127) / 128 + epi.sw_width / 64);
+  run_rows(m, n, k, [&](int64_t row0, int64_t rows, int tile) {
     Epilogue e = epi;
     e.rows_desc = rows_last_first(rows, k);
     e.row0 = row0;
     if (epi.c2) e.c2 = static_cast<uint16_t*>(epi.c2) + row0 * epi.ldc2;
     const Call x{a + row0 * lda, lda, w, ldw, static_cast<uint16_t*>(c) + row0 * ldc, ldc, (int)rows, n, k, 1, s};
-    if (tile == DT256x256) run_pp<256, 0, false, true, false>(x, e, tiles_n);
-    else run_pp<128, 0, false, true, false>(x, e, tiles_n);
+    run_tile<0, false, true, false>(tile, x, e, t256, t128);
   });
 }
 

@@ -37,7 +37,7 @@ import torch
 from .. import _lib
 from ..kernels import fused_ops
 from ..ltx2 import dense_attention as _dense
-from ..ltx2.attention import Linear, _cat_layers, qknorm_rope_projection
+from ..ltx2.attention import Linear, _cat_layers, qknorm_rope_projection, swiglu_projection
 from ..ltx2.transformer import layer_norm_modulate
 from .kv import attend
 
@@ -146,10 +146,13 @@ class FeedForward:
 
     def __call__(self, value: torch.Tensor, *, residual: torch.Tensor | None = None,
                  gate: torch.Tensor | None = None, out_dtype: torch.dtype | None = None) -> torch.Tensor:
-        """With ``residual``/``gate`` the block's ``residual + gate * ff(x)`` is formed in the
-        ``linear_out`` epilogue, written as ``out_dtype`` (default the input dtype)."""
-        return self.linear_out(fused_ops.swiglu(self.linear_in(value)), residual=residual, gate=gate,
-                               out_dtype=out_dtype)
+        """The SwiGLU is formed in the ``linear_in`` epilogue where the layer allows it. With
+        ``residual``/``gate`` the block's ``residual + gate * ff(x)`` is formed in the ``linear_out``
+        epilogue, written as ``out_dtype`` (default the input dtype)."""
+        hidden = swiglu_projection(self.linear_in, value)
+        if hidden is None:
+            hidden = fused_ops.swiglu(self.linear_in(value))
+        return self.linear_out(hidden, residual=residual, gate=gate, out_dtype=out_dtype)
 
 
 def _norm_rope_into(raw: torch.Tensor, out: torch.Tensor, norm: QKNorm, cos: torch.Tensor, sin: torch.Tensor,
@@ -241,7 +244,7 @@ class DoubleAttention:
                     and qknorm_rope_projection(fused, value[b], rows[b], q_width=width, k_width=width,
                                                norm_q=norm_q.weight, norm_k=norm_k.weight, eps=1e-6,
                                                weight_offset=0.0, cos=cos[tb, row0:row0 + count, 0],
-                                               sin=sin[tb, row0:row0 + count, 0])):
+                                               sin=sin[tb, row0:row0 + count, 0], head_dim=self.head_dim)):
                 continue
             entry = rows[b:b + 1]
             self._project(fused, layers, value[b:b + 1], entry)
@@ -338,23 +341,27 @@ class SingleAttention:
         if mlp_width <= 0 or mlp_width % 2:
             raise ValueError(f"to_qkv_mlp_proj width {total} does not split into [{width} x 3, 2F]")
         cos, sin = _tables(positions, batch, tokens, self.head_dim)
-        fused = torch.empty((batch, tokens, total), dtype=torch.bfloat16, device=value.device)
+        inner = mlp_width // 2
+        joined = torch.empty((batch, tokens, width + inner), dtype=torch.bfloat16, device=value.device)
+        qkv = torch.empty((batch, tokens, 3 * width), dtype=torch.bfloat16, device=value.device)
         if (self.norm_q.weight is not None and self.norm_k.weight is not None and value.is_contiguous()
                 and qknorm_rope_projection(self.to_qkv_mlp_proj, value.view(batch * tokens, -1),
-                                           fused.view(batch * tokens, total), q_width=width, k_width=width,
+                                           qkv.view(batch * tokens, 3 * width), q_width=width, k_width=width,
                                            norm_q=self.norm_q.weight, norm_k=self.norm_k.weight, eps=1e-6,
-                                           weight_offset=0.0, cos=cos[:, :, 0], sin=sin[:, :, 0])):
-            q, k = fused[..., :width], fused[..., width:2 * width]
-        else:  # the projection, then the norm + RoPE pass
+                                           weight_offset=0.0, cos=cos[:, :, 0], sin=sin[:, :, 0],
+                                           head_dim=self.head_dim,
+                                           swiglu_out=joined.view(batch * tokens, -1)[:, width:])):
+            # one GEMM: Q and K normalized and rotated, the MLP half already silu(gate) * up beside the
+            # attention output's columns
+            q, k, v = qkv[..., :width], qkv[..., width:2 * width], qkv[..., 2 * width:]
+        else:  # the projection, then the norm + RoPE and SwiGLU passes
+            fused = torch.empty((batch, tokens, total), dtype=torch.bfloat16, device=value.device)
             self.to_qkv_mlp_proj(value, out=fused)
-            q = torch.empty((batch, tokens, width), dtype=torch.bfloat16, device=value.device)
-            k = torch.empty_like(q)
+            q, k, v = qkv[..., :width], qkv[..., width:2 * width], fused[..., 2 * width:3 * width]
             _norm_rope_into(fused[..., :width], q, self.norm_q, cos, sin, 0, self.heads)
             _norm_rope_into(fused[..., width:2 * width], k, self.norm_k, cos, sin, 0, self.heads)
-        joined = torch.empty((batch, tokens, width + mlp_width // 2), dtype=torch.bfloat16, device=value.device)
-        _dense.batched_attention(q, k, fused[..., 2 * width:3 * width], heads=self.heads,
-                                     scale=self.head_dim ** -0.5, out=joined[..., :width])
-        _lib.launch_swiglu(fused[..., 3 * width:], joined[..., width:])
+            _lib.launch_swiglu(fused[..., 3 * width:], joined[..., width:])
+        _dense.batched_attention(q, k, v, heads=self.heads, scale=self.head_dim ** -0.5, out=joined[..., :width])
         return self.to_out(joined, residual=residual, gate=gate, out_dtype=out_dtype)
 
 

@@ -32,7 +32,7 @@ import torch
 from .. import _lib
 from ..kernels import fused_ops
 from ..ltx2 import dense_attention as _dense
-from ..ltx2.attention import Linear, _cat_layers, qknorm_rope_projection
+from ..ltx2.attention import Linear, _cat_layers, qknorm_rope_projection, swiglu_projection
 from ..ltx2.transformer import adaln
 
 __all__ = [
@@ -251,6 +251,9 @@ class Krea2SwiGLU:
                  residual_gate: torch.Tensor | None = None, out_dtype: torch.dtype | None = None) -> torch.Tensor:
         if hidden_states.shape[-1] != self.hidden_size:
             raise ValueError(f"Krea SwiGLU expects width {self.hidden_size}, got {hidden_states.shape[-1]}")
+        hidden = None if self._gate_up is None else swiglu_projection(self._gate_up, hidden_states)
+        if hidden is not None:
+            return self.down(hidden, residual=residual, gate=residual_gate, out_dtype=out_dtype)
         if self._gate_up is not None:
             both = self._gate_up(hidden_states)
         else:  # the two products side by side in one buffer, as the fused weight writes them

@@ -21,7 +21,7 @@ import torch
 
 from .. import _lib
 from ..kernels import fused_ops, mpp_linear, split_rope
-from ..kernels.quantized import PretransposedQuantizedLinear, QuantizedLinear
+from ..kernels.quantized import PretransposedQuantizedLinear, QuantizedLinear, dequant_workspace
 from . import dense_attention as _dense
 from .rope import LTXRopeType
 
@@ -202,43 +202,86 @@ def _dense_weight(layer):
     if isinstance(layer, PretransposedQuantizedLinear):
         return layer._dense
     if isinstance(layer, QuantizedLinear) and layer.weight.is_cuda:
-        return layer._dense if layer._dense is not None else layer.dequantized()
+        if layer._dense is not None:
+            return layer._dense
+        return layer.dequantized(dequant_workspace(layer.out_features, layer.in_features, layer.weight.device))
     return None
+
+
+def _gemm_rows(value: torch.Tensor) -> torch.Tensor:
+    """``value``'s rows as the GEMMs read them: ``(R, in)``, 16-byte aligned."""
+    a = value.reshape(-1, value.shape[-1])
+    return a if a.stride(-1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 else a.contiguous()
+
+
+def swiglu_projection(layer, value: torch.Tensor) -> torch.Tensor | None:
+    """``silu(gate) * up`` of ``[gate | up] = layer(value)``, the product formed in the GEMM's epilogue
+    (``kx_gemm_columns_bf16``): the two halves are never stored and are multiplied before their one
+    rounding. None (nothing ran) when the layer or the shapes do not take this path; the caller then
+    runs the projection and the SwiGLU pass."""
+    weight = _dense_weight(layer) if value.is_cuda and value.dtype == torch.bfloat16 else None
+    if weight is None or weight.dtype != torch.bfloat16 or value.numel() == 0:
+        return None
+    n, k = (int(s) for s in weight.shape)
+    bias = getattr(layer, "bias", None)
+    if (n % 256 or k % 64 or int(value.shape[-1]) != k or weight.stride(1) != 1 or weight.stride(0) % 8
+            or weight.stride(0) > 1 << 22 or weight.data_ptr() % 16 or (n // 2 + 256) * weight.stride(0) * 2 >= 1 << 32):
+        return None
+    a = _gemm_rows(value)
+    if a.stride(0) > 1 << 22:
+        return None
+    out = torch.empty((*value.shape[:-1], n // 2), dtype=torch.bfloat16, device=value.device)
+    _lib.launch_gemm_columns(a, weight, None, bias=None if bias is None else bias.to(torch.bfloat16).contiguous(),
+                             swiglu_begin=0, swiglu_out=out.view(-1, n // 2))
+    return out
 
 
 def qknorm_rope_projection(layer, value: torch.Tensor, out: torch.Tensor, *, q_width: int, k_width: int,
                            norm_q: torch.Tensor, norm_k: torch.Tensor, eps: float, weight_offset: float,
-                           cos: torch.Tensor, sin: torch.Tensor) -> bool:
+                           cos: torch.Tensor, sin: torch.Tensor, head_dim: int = 128,
+                           swiglu_out: torch.Tensor | None = None) -> bool:
     """``out = layer(value)`` with the query columns ``[0, q_width)`` and key columns
-    ``[q_width, q_width + k_width)`` normalized per 128-wide head (``(x * rsqrt(mean(x^2) + eps))
-    * (w + weight_offset)`` of the bf16 projection) and rotated in adjacent pairs, all in the GEMM's
-    epilogue (``kx_gemm_qknorm_rope_bf16``). ``value`` ``(R, in)`` and ``out`` ``(R, out)`` are the
-    rows of ``R / T`` sequences of ``T`` tokens; ``cos``/``sin`` are their fp32 tables, ``(T, 128)``
-    or ``(1 | R / T, T, 128)``, with unit-stride rows. Returns False (nothing written) when the layer
-    or the shapes do not take this path; the caller then runs the separate passes."""
+    ``[q_width, q_width + k_width)`` normalized per ``head_dim``-wide head (64 or 128;
+    ``(x * rsqrt(mean(x^2) + eps)) * (w + weight_offset)`` of the bf16 projection) and rotated in
+    adjacent pairs, all in the GEMM's epilogue (``kx_gemm_columns_bf16``). ``value`` ``(R, in)`` and
+    ``out`` are the rows of ``R / T`` sequences of ``T`` tokens; ``cos``/``sin`` are their fp32 tables,
+    ``(T, head_dim)`` or ``(1 | R / T, T, head_dim)``, with unit-stride rows. With ``swiglu_out``
+    ``(R, F)`` the layer's last ``2 F`` columns are a SwiGLU pair that goes there, and ``out`` holds the
+    columns before them. Returns False (nothing written) when the layer or the shapes do not take
+    this path; the caller then runs the separate passes."""
+    if value.dtype != torch.bfloat16 or value.dim() != 2 or out.dim() != 2 or cos.dim() not in (2, 3) \
+            or cos.shape != sin.shape or cos.stride() != sin.stride() or head_dim not in (64, 128):
+        return False
     weight = _dense_weight(layer)
-    if (weight is None or weight.dtype != torch.bfloat16 or value.dtype != torch.bfloat16 or value.dim() != 2
-            or out.dim() != 2 or cos.dim() not in (2, 3) or cos.shape != sin.shape or cos.stride() != sin.stride()):
+    if weight is None or weight.dtype != torch.bfloat16:
         return False
     rows, k = int(value.shape[0]), int(value.shape[1])
     n = int(weight.shape[0])
+    begin = n if swiglu_out is None else n - 2 * int(swiglu_out.shape[-1])
     tokens = int(cos.shape[-2])
     batches = 1 if cos.dim() == 2 else int(cos.shape[0])
-    if (rows == 0 or tokens == 0 or rows % tokens or batches not in (1, rows // tokens) or cos.shape[-1] != 128
-            or q_width % 128 or k_width % 128 or q_width + k_width > n or k % 64 or int(weight.shape[1]) != k
-            or norm_q.shape != (128,) or norm_k.shape != (128,) or norm_q.dtype != norm_k.dtype
+    if (rows == 0 or tokens == 0 or rows % tokens or batches not in (1, rows // tokens) or cos.shape[-1] != head_dim
+            or q_width % 128 or k_width % 128 or q_width + k_width > begin or k % 64 or int(weight.shape[1]) != k
+            or norm_q.shape != (head_dim,) or norm_k.shape != (head_dim,) or norm_q.dtype != norm_k.dtype
+            or norm_q.dtype not in (torch.float32, torch.bfloat16)
             or cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.stride(-1) != 1
             or cos.stride(-2) % 4 or (batches > 1 and cos.stride(0) % 4) or cos.data_ptr() % 16
-            or sin.data_ptr() % 16 or tuple(out.shape) != (rows, n) or out.dtype != torch.bfloat16
+            or sin.data_ptr() % 16 or tuple(out.shape) != (rows, begin) or out.dtype != torch.bfloat16
             or out.stride(-1) != 1 or out.stride(0) % 4 or out.data_ptr() % 8):
         return False
-    a = value if value.stride(-1) == 1 and value.stride(0) % 8 == 0 and value.data_ptr() % 16 == 0 else value.contiguous()
+    if swiglu_out is not None and (begin < 0 or begin % 256 or (n - begin) % 256 or swiglu_out.dim() != 2
+                                   or swiglu_out.dtype != torch.bfloat16 or int(swiglu_out.shape[0]) != rows
+                                   or swiglu_out.stride(-1) != 1 or swiglu_out.stride(0) % 4
+                                   or swiglu_out.data_ptr() % 8 or ((n - begin) // 2 + 256) * k * 2 >= 1 << 32):
+        return False
     bias = getattr(layer, "bias", None)
-    bias = None if bias is None else bias.to(torch.bfloat16).contiguous()
-    _lib.launch_gemm_qknorm_rope(a, weight, out, bias=bias, q_end=q_width, k_end=q_width + k_width,
-                                 norm_q=norm_q.contiguous(), norm_k=norm_k.contiguous(), eps=eps,
-                                 weight_offset=weight_offset, cos=cos, sin=sin, table_ld=int(cos.stride(-2)),
-                                 table_hs=0, table_rows=tokens, table_bs=int(cos.stride(0)) if batches > 1 else 0)
+    _lib.launch_gemm_columns(_gemm_rows(value), weight, out,
+                             bias=None if bias is None else bias.to(torch.bfloat16).contiguous(), q_end=q_width,
+                             k_end=q_width + k_width, head_dim=head_dim, norm_q=norm_q.contiguous(),
+                             norm_k=norm_k.contiguous(), eps=eps, weight_offset=weight_offset, cos=cos, sin=sin,
+                             table_ld=int(cos.stride(-2)), table_hs=0, table_rows=tokens,
+                             table_bs=int(cos.stride(0)) if batches > 1 else 0, swiglu_begin=begin,
+                             swiglu_out=swiglu_out)
     return True
 
 
@@ -348,4 +391,5 @@ __all__ = [
     "qknorm_rope_projection",
     "rms_norm",
     "scaled_dot_product_attention",
+    "swiglu_projection",
 ]
