@@ -192,6 +192,14 @@ int kx_qk_rmsnorm_rope_bf16(const void* xq, int64_t ldq, const void* xk, int64_t
                             int64_t table_ld, int64_t table_hs, int64_t tokens, int table_batched,
                             kx_stream_t stream);
 
+/* The same pass for 64-wide heads (the audio stream's self-attention). */
+int kx_qk_rmsnorm_rope_h64_bf16(const void* xq, int64_t ldq, const void* xk, int64_t ldk, void* yq,
+                                int64_t ldyq, void* yk, int64_t ldyk, int64_t rows, int64_t dim,
+                                const void* wq, const void* wk, int w_dtype, float eps,
+                                float weight_offset, const float* cos, const float* sin,
+                                int64_t table_ld, int64_t table_hs, int64_t tokens, int table_batched,
+                                kx_stream_t stream);
+
 /*
  * Dense bf16 linear on MFMA: c = epilogue(a · wᵀ) with fp32 accumulation and one rounding.
  * Replaces mpp_linear.linear / mx.addmm(bias, x, Wᵀ) (kinomlx/kernels/mpp_linear.py:469-506,
@@ -418,6 +426,15 @@ int kx_table_add_f32(const void* table, int table_dtype, const void* ts, int ts_
                      int64_t ts_ts, int64_t ts_rs, float* out, int64_t batch, int64_t tokens, int64_t rows,
                      int64_t dim, int round_dtype, kx_stream_t stream);
 
+/* A Krea 2 block's six modulation rows: out[r, i, c] = fp32(projected[r, i * dim + c]) +
+ * fp32(table[i, c]) for i < 6 (fp32 (rows, 6, dim) contiguous; projected rows ldp elements apart), the
+ * two scale rows with the zero-centred norm weight they multiply folded in: row 0 becomes
+ * (1 + row) (1 + w1) - 1 and row 3 (1 + row) (1 + w2) - 1. split_six_way_modulation and the norms'
+ * weights (kinomlx/models/krea2/transformer/model.py:29-46,288-307,327-348). */
+int kx_six_way_modulation_f32(const void* projected, int p_dtype, int64_t ldp, const void* table, int t_dtype,
+                              const float* w1, const float* w2, float* out, int64_t rows, int64_t dim,
+                              kx_stream_t stream);
+
 /* tanh GELU in fp32, inner argument clamped to +-10: fused_ops.gelu_approx
  * (kinomlx/kernels/fused_ops.py:27-35,327-350). */
 int kx_gelu_tanh_bf16(const void* x, void* y, int64_t count, kx_stream_t stream);
@@ -517,6 +534,11 @@ int kx_qk_rmsnorm_rope_f16(const void* xq, int64_t ldq, const void* xk, int64_t 
                            int w_dtype, float eps, float weight_offset, const float* cos, const float* sin,
                            int64_t table_ld, int64_t table_hs, int64_t tokens, int table_batched,
                            kx_stream_t stream);
+int kx_qk_rmsnorm_rope_h64_f16(const void* xq, int64_t ldq, const void* xk, int64_t ldk, void* yq, int64_t ldyq,
+                               void* yk, int64_t ldyk, int64_t rows, int64_t dim, const void* wq, const void* wk,
+                               int w_dtype, float eps, float weight_offset, const float* cos, const float* sin,
+                               int64_t table_ld, int64_t table_hs, int64_t tokens, int table_batched,
+                               kx_stream_t stream);
 int kx_rope_split_f16(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t batch, int64_t tokens,
                       int64_t heads, int64_t half, const float* cos, const float* sin, int table_batched,
                       kx_stream_t stream);

@@ -60,6 +60,10 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _I, _F, _F, _P, _P, _I64, _I64, _I64, _I,
         _P,
     ],
+    "kx_qk_rmsnorm_rope_h64_bf16": [
+        _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _I, _F, _F, _P, _P, _I64, _I64, _I64, _I,
+        _P,
+    ],
     "kx_rope_split_bf16": [_P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _I, _P],
     "kx_rope_pair_bf16": [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64, _I64, _I, _P],
     "kx_attention_fwd_bf16": [
@@ -97,6 +101,7 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P, _I64, _P, _I64, _I64, _P,
     ],
     "kx_table_add_f32": [_P, _I, _P, _I, _I64, _I64, _I64, _P, _I64, _I64, _I64, _I64, _I, _P],
+    "kx_six_way_modulation_f32": [_P, _I, _I64, _P, _I, _P, _P, _P, _I64, _I64, _P],
     "kx_gemm_qknorm_rope_bf16": [
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I, _F, _F, _P, _P, _I64, _I64,
         _I64, _I64, _P,
@@ -128,7 +133,7 @@ SIGNATURES: dict[str, list] = {
 
 # fp16 entry points: the bf16 namesake's arguments with fp16 16-bit tensors (include/kx355.h)
 F16_ENTRIES = (
-    "kx_adaln_norm", "kx_rmsnorm_rope", "kx_qk_rmsnorm_rope", "kx_rope_split", "kx_rope_pair",
+    "kx_adaln_norm", "kx_rmsnorm_rope", "kx_qk_rmsnorm_rope", "kx_qk_rmsnorm_rope_h64", "kx_rope_split", "kx_rope_pair",
     "kx_attention_fwd", "kx_attention_gqa_fwd", "kx_attention_bias_fwd", "kx_attention_split_fwd", "kx_gemm",
     "kx_gemm_splitk", "kx_gelu_tanh", "kx_silu", "kx_swiglu", "kx_modulate", "kx_gated_residual",
 )
@@ -340,7 +345,7 @@ def launch_rmsnorm_rope(
 
 
 def launch_qk_rmsnorm_rope(xq, xk, yq, yk, wq, wk, eps: float, *, cos, sin, table_ld: int, table_hs: int,
-                           tokens: int, table_batched: bool) -> bool:
+                           tokens: int, table_batched: bool, head_dim: int = 128) -> bool:
     """One pass for the Q and K rows of the same tokens; False (nothing launched) when the shape
     or alignment is outside the fused kernel's contract."""
     _check_gpu("qk_rmsnorm_rope", xq, xk, yq, yk, wq, wk, cos, sin)
@@ -354,7 +359,7 @@ def launch_qk_rmsnorm_rope(xq, xk, yq, yk, wq, wk, eps: float, *, cos, sin, tabl
     _same_dtype("qk_rmsnorm_rope", xq.dtype, xk, yq, yk)
     w_dtype = _weight_code(wq, "rms_norm")
     code = _call(
-        f"kx_qk_rmsnorm_rope_{suffix}", _ptr(xq), ldq, _ptr(xk), ldk, _ptr(yq), ldyq, _ptr(yk), ldyk, rows, dim,
+        f"kx_qk_rmsnorm_rope_{'h64_' if head_dim == 64 else ''}{suffix}", _ptr(xq), ldq, _ptr(xk), ldk, _ptr(yq), ldyq, _ptr(yk), ldyk, rows, dim,
         _ptr(wq), _ptr(wk), w_dtype, eps, 0.0, _ptr(cos), _ptr(sin), table_ld, table_hs, tokens,
         int(table_batched), _stream(), unsupported_ok=True,
     )
@@ -807,6 +812,24 @@ def table_add(table: torch.Tensor, ts: torch.Tensor | None, round_to: torch.dtyp
     out = torch.empty((batch, tokens, rows, dim), dtype=torch.float32, device=table.device)
     _call("kx_table_add_f32", _ptr(table), _weight_code(table, "table_add table"), _ptr(ts), ts_code, bs, tstride, rs,
           _ptr(out), batch, tokens, rows, dim, round_code, _stream())
+    return out
+
+
+def six_way_modulation(projected: torch.Tensor, table: torch.Tensor, w1: torch.Tensor,
+                       w2: torch.Tensor) -> torch.Tensor:
+    """``projected (..., 6 D) + table (6, D)`` as fp32 ``(..., 6, D)``, rows 0 and 3 (the scales) with the
+    zero-centred norm weights ``w1`` and ``w2`` ``(D,)`` folded in: ``(1 + scale) (1 + w) - 1``."""
+    dim = int(table.shape[1])
+    projected = projected if projected.is_contiguous() else projected.contiguous()
+    table = table if table.is_contiguous() else table.contiguous()
+    w1, w2 = (w.float().contiguous() for w in (w1, w2))
+    _check_gpu("six_way_modulation", projected, table, w1, w2)
+    if w1.shape != (dim,) or w2.shape != (dim,):
+        raise ValueError(f"six_way_modulation: norm weights must have shape ({dim},)")
+    out = torch.empty((*projected.shape[:-1], 6, dim), dtype=torch.float32, device=projected.device)
+    _call("kx_six_way_modulation_f32", _ptr(projected), _weight_code(projected, "six_way_modulation"), 6 * dim,
+          _ptr(table), _weight_code(table, "six_way_modulation table"), _ptr(w1), _ptr(w2), _ptr(out),
+          projected.numel() // (6 * dim), dim, _stream())
     return out
 
 

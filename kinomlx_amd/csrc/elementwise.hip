@@ -30,16 +30,26 @@ __global__ __launch_bounds__(256) void unary_scalar(const uint16_t* __restrict__
   y[i] = f2e<H>(act<OP>(e2f<H>(x[i])));
 }
 
-template <bool H>
+// V columns per thread (8 where 16-byte accesses fit, else 1).
+template <bool H, int V>
 __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                      uint16_t* __restrict__ y, int64_t ldy,
                                                      int64_t rows, int64_t hidden) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows * hidden) return;
-  const int64_t r = i / hidden, c = i - r * hidden;
-  const float g = e2f<H>(x[r * ldx + c]);
-  const float u = e2f<H>(x[r * ldx + hidden + c]);
-  y[r * ldy + c] = f2e<H>(silu(g) * u);
+  const int64_t per_row = hidden / V;
+  if (i >= rows * per_row) return;
+  const int64_t r = i / per_row, c = (i - r * per_row) * V;
+  const uint16_t* xr = x + r * ldx + c;
+  if constexpr (V == 8) {
+    float g[8], u[8];
+    e_unpack8<H>(*reinterpret_cast<const uint4*>(xr), g);
+    e_unpack8<H>(*reinterpret_cast<const uint4*>(xr + hidden), u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) g[j] = silu(g[j]) * u[j];
+    *reinterpret_cast<uint4*>(y + r * ldy + c) = e_pack8<H>(g);
+  } else {
+    y[r * ldy + c] = f2e<H>(silu(e2f<H>(*xr)) * e2f<H>(xr[hidden]));
+  }
 }
 
 // fp32 of element i of an fp32, bf16 or fp16 array (dtype code DT)
@@ -85,8 +95,12 @@ int swiglu(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, int64
   KX_REQUIRE(x && y && rows >= 0 && hidden > 0 && ldx >= 2 * hidden && ldy >= hidden, "%s: bad argument", name);
   const int64_t total = rows * hidden;
   if (total == 0) return KX_OK;
-  swiglu_kernel<H><<<(unsigned)((total + 255) / 256), 256, 0, s>>>((const uint16_t*)x, ldx, (uint16_t*)y, ldy,
-                                                                  rows, hidden);
+  if (hidden % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y))
+    swiglu_kernel<H, 8><<<(unsigned)((total / 8 + 255) / 256), 256, 0, s>>>((const uint16_t*)x, ldx, (uint16_t*)y, ldy,
+                                                                           rows, hidden);
+  else
+    swiglu_kernel<H, 1><<<(unsigned)((total + 255) / 256), 256, 0, s>>>((const uint16_t*)x, ldx, (uint16_t*)y, ldy,
+                                                                       rows, hidden);
   return check_launch(name);
 }
 

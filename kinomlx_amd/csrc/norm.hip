@@ -139,6 +139,18 @@ __device__ __forceinline__ float load_w(const void* w, int64_t i) {
   else return reinterpret_cast<const float*>(w)[i];
 }
 
+// Eight consecutive weights from column i (a multiple of 8): vector loads where the weight is 16-byte
+// aligned (vec), the same values one by one where it is a view at another offset.
+template <int WT>
+__device__ __forceinline__ void load_w8(const void* w, int64_t i, bool vec, float* v) {
+  if (vec) {
+    load8<WT == KX_F16, WT == KX_F32>(w, i, v);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = load_w<WT>(w, i + j);
+  }
+}
+
 template <bool H, int VPL, int G, int ROPE, int WT>
 __global__ __launch_bounds__(256) void rmsnorm_rope_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy,
@@ -180,9 +192,10 @@ __global__ __launch_bounds__(256) void rmsnorm_rope_kernel(
   for (int i = 0; i < VPL; ++i) {
     const int col = (i * 64 + lane) * 8;
     const int wcol = (G == 0) ? col : (col % norm_width);
+    float wv[8];
+    load_w8<WT>(w, wcol, (reinterpret_cast<uintptr_t>(w) & 15) == 0, wv);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[i][j] = v[i][j] * inv[i] * (load_w<WT>(w, wcol + j) + weight_offset);
+    for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * inv[i] * (wv[j] + weight_offset);
   }
   uint16_t* yr = y + row * ldy;
   if (ROPE == KX_ROPE_NONE) {
@@ -242,15 +255,50 @@ __global__ __launch_bounds__(256) void rmsnorm_rope_kernel(
   }
 }
 
-// Full-width weighted RMSNorm with split-half RoPE for 128-wide heads (the LTX q/k path): each
-// lane owns matching 8-value chunks of both halves of a head (dims d .. d+7 and d+64 .. d+71), so
-// the rotation needs no lane exchange and every cos / sin table value is read once. All loads
-// (row, both tables) are issued before the row reduction. Rounding as rmsnorm_rope_kernel: the
-// normalized value stays fp32, each RoPE product is rounded before the difference / sum.
-template <bool H, int VPL, int WT>
-__global__ __launch_bounds__(256) void rmsnorm_rope_split128_kernel(
+// Full-width weighted RMSNorm with split-half RoPE for heads of 2 HALF columns (HALF = 64: the LTX
+// video q/k path; 32: the audio and A/V paths): each lane owns matching 8-value chunks of both halves
+// of a head (dims d .. d+7 and d+HALF .. d+HALF+7), so the rotation needs no lane exchange and every
+// cos / sin table value is read once, by 16-byte loads. All loads (row, both tables) are issued before
+// the row reduction. Rounding as rmsnorm_rope_kernel: the normalized value stays fp32, each RoPE
+// product is rounded before the difference / sum.
+template <int HALF>
+struct SplitChunk {
+  int head, k, col;  // head, chunk within its half, first column
+  __device__ __forceinline__ explicit SplitChunk(int p) : head(p / (HALF / 8)), k(p % (HALF / 8)) {
+    col = head * 2 * HALF + k * 8;
+  }
+};
+__device__ __forceinline__ void load_f8(const float* p, float* v) {
+  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+// One chunk pair normalized by r, weighted and rotated, to yr + col and yr + col + HALF.
+template <bool H, int HALF, int WT>
+__device__ __forceinline__ void split_rotate(const float* a, const float* b, float r, const void* w, bool wvec,
+                                             float weight_offset, const float* c, const float* sn, uint16_t* yr,
+                                             int col) {
+  float w0[8], w1[8], o0[8], o1[8];
+  load_w8<WT>(w, col, wvec, w0);
+  load_w8<WT>(w, col + HALF, wvec, w1);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+#pragma clang fp contract(off)
+    const float n0 = a[j] * r * (w0[j] + weight_offset);
+    const float n1 = b[j] * r * (w1[j] + weight_offset);
+    const float fc = n0 * c[j], ss2 = n1 * sn[j];  // first * c, second * s
+    const float fs = n0 * sn[j], sc = n1 * c[j];   // first * s, second * c
+    o0[j] = fc - ss2;
+    o1[j] = fs + sc;
+  }
+  *reinterpret_cast<uint4*>(yr + col) = e_pack8<H>(o0);
+  *reinterpret_cast<uint4*>(yr + col + HALF) = e_pack8<H>(o1);
+}
+
+template <bool H, int HALF, int VPL, int WT>
+__global__ __launch_bounds__(256) void rmsnorm_rope_split_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy,
-    int64_t rows, const void* __restrict__ w, float eps, float weight_offset,
+    int64_t rows, const void* __restrict__ w, bool wvec, float eps, float weight_offset,
     const float* __restrict__ cosp, const float* __restrict__ sinp, int64_t table_ld,
     int64_t table_hs, int64_t tokens, int table_batched) {
   constexpr int DIM = VPL * 512;
@@ -263,18 +311,11 @@ __global__ __launch_bounds__(256) void rmsnorm_rope_split128_kernel(
   float a[NP][8], b[NP][8], c[NP][8], sn[NP][8];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const int p = i * 64 + lane, h = p >> 3, k = p & 7;
-    const int col = h * 128 + k * 8;
-    e_unpack8<H>(*reinterpret_cast<const uint4*>(xr + col), a[i]);
-    e_unpack8<H>(*reinterpret_cast<const uint4*>(xr + col + 64), b[i]);
-    const float* cr = cosp + tok * table_ld + h * table_hs + k * 8;
-    const float* sr = sinp + tok * table_ld + h * table_hs + k * 8;
-    const float4 c0 = *reinterpret_cast<const float4*>(cr), c1 = *reinterpret_cast<const float4*>(cr + 4);
-    const float4 s0 = *reinterpret_cast<const float4*>(sr), s1 = *reinterpret_cast<const float4*>(sr + 4);
-    c[i][0] = c0.x; c[i][1] = c0.y; c[i][2] = c0.z; c[i][3] = c0.w;
-    c[i][4] = c1.x; c[i][5] = c1.y; c[i][6] = c1.z; c[i][7] = c1.w;
-    sn[i][0] = s0.x; sn[i][1] = s0.y; sn[i][2] = s0.z; sn[i][3] = s0.w;
-    sn[i][4] = s1.x; sn[i][5] = s1.y; sn[i][6] = s1.z; sn[i][7] = s1.w;
+    const SplitChunk<HALF> p(i * 64 + lane);
+    e_unpack8<H>(*reinterpret_cast<const uint4*>(xr + p.col), a[i]);
+    e_unpack8<H>(*reinterpret_cast<const uint4*>(xr + p.col + HALF), b[i]);
+    load_f8(cosp + tok * table_ld + p.head * table_hs + p.k * 8, c[i]);
+    load_f8(sinp + tok * table_ld + p.head * table_hs + p.k * 8, sn[i]);
   }
   float ss = 0.0f;
 #pragma unroll
@@ -282,36 +323,21 @@ __global__ __launch_bounds__(256) void rmsnorm_rope_split128_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j) ss = fmaf(b[i][j], b[i][j], fmaf(a[i][j], a[i][j], ss));
   const float r = rsqrtf(wave_sum<64>(ss) * (1.0f / DIM) + eps);
-  uint16_t* yr = y + row * ldy;
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int p = i * 64 + lane, h = p >> 3, k = p & 7;
-    const int col = h * 128 + k * 8;
-    float o0[8], o1[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-#pragma clang fp contract(off)
-      const float n0 = a[i][j] * r * (load_w<WT>(w, col + j) + weight_offset);
-      const float n1 = b[i][j] * r * (load_w<WT>(w, col + 64 + j) + weight_offset);
-      const float fc = n0 * c[i][j], ss2 = n1 * sn[i][j];  // first * c, second * s
-      const float fs = n0 * sn[i][j], sc = n1 * c[i][j];   // first * s, second * c
-      o0[j] = fc - ss2;
-      o1[j] = fs + sc;
-    }
-    *reinterpret_cast<uint4*>(yr + col) = e_pack8<H>(o0);
-    *reinterpret_cast<uint4*>(yr + col + 64) = e_pack8<H>(o1);
-  }
+  for (int i = 0; i < NP; ++i)
+    split_rotate<H, HALF, WT>(a[i], b[i], r, w, wvec, weight_offset, c[i], sn[i], y + row * ldy,
+                              SplitChunk<HALF>(i * 64 + lane).col);
 }
 
 // Q and K of the same tokens in one pass (self-attention q_norm / k_norm + split RoPE): a wave
 // handles one token's Q row and K row with their own weights and shares the token's cos / sin
 // table values between them, so the tables (as large as Q and K together at D = 4096, fp32) are
-// read once instead of twice. Per row the arithmetic is exactly rmsnorm_rope_split128_kernel's.
-template <bool H, int VPL, int WT>
-__global__ __launch_bounds__(256) void qk_rmsnorm_rope_split128_kernel(
+// read once instead of twice. Per row the arithmetic is exactly rmsnorm_rope_split_kernel's.
+template <bool H, int HALF, int VPL, int WT>
+__global__ __launch_bounds__(256) void qk_rmsnorm_rope_split_kernel(
     const uint16_t* __restrict__ xq, int64_t ldq, const uint16_t* __restrict__ xk, int64_t ldk,
     uint16_t* __restrict__ yq, int64_t ldyq, uint16_t* __restrict__ yk, int64_t ldyk, int64_t rows,
-    const void* __restrict__ wq, const void* __restrict__ wk, float eps, float weight_offset,
+    const void* __restrict__ wq, const void* __restrict__ wk, bool wvec, float eps, float weight_offset,
     const float* __restrict__ cosp, const float* __restrict__ sinp, int64_t table_ld,
     int64_t table_hs, int64_t tokens, int table_batched) {
   constexpr int DIM = VPL * 512;
@@ -324,20 +350,13 @@ __global__ __launch_bounds__(256) void qk_rmsnorm_rope_split128_kernel(
   float c[NP][8], sn[NP][8];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const int p = i * 64 + lane, h = p >> 3, k = p & 7;
-    const int col = h * 128 + k * 8;
-    qa[i] = *reinterpret_cast<const uint4*>(xq + row * ldq + col);
-    qb[i] = *reinterpret_cast<const uint4*>(xq + row * ldq + col + 64);
-    ka[i] = *reinterpret_cast<const uint4*>(xk + row * ldk + col);
-    kb[i] = *reinterpret_cast<const uint4*>(xk + row * ldk + col + 64);
-    const float* cr = cosp + tok * table_ld + h * table_hs + k * 8;
-    const float* sr = sinp + tok * table_ld + h * table_hs + k * 8;
-    const float4 c0 = *reinterpret_cast<const float4*>(cr), c1 = *reinterpret_cast<const float4*>(cr + 4);
-    const float4 s0 = *reinterpret_cast<const float4*>(sr), s1 = *reinterpret_cast<const float4*>(sr + 4);
-    c[i][0] = c0.x; c[i][1] = c0.y; c[i][2] = c0.z; c[i][3] = c0.w;
-    c[i][4] = c1.x; c[i][5] = c1.y; c[i][6] = c1.z; c[i][7] = c1.w;
-    sn[i][0] = s0.x; sn[i][1] = s0.y; sn[i][2] = s0.z; sn[i][3] = s0.w;
-    sn[i][4] = s1.x; sn[i][5] = s1.y; sn[i][6] = s1.z; sn[i][7] = s1.w;
+    const SplitChunk<HALF> p(i * 64 + lane);
+    qa[i] = *reinterpret_cast<const uint4*>(xq + row * ldq + p.col);
+    qb[i] = *reinterpret_cast<const uint4*>(xq + row * ldq + p.col + HALF);
+    ka[i] = *reinterpret_cast<const uint4*>(xk + row * ldk + p.col);
+    kb[i] = *reinterpret_cast<const uint4*>(xk + row * ldk + p.col + HALF);
+    load_f8(cosp + tok * table_ld + p.head * table_hs + p.k * 8, c[i]);
+    load_f8(sinp + tok * table_ld + p.head * table_hs + p.k * 8, sn[i]);
   }
   float ssq = 0.0f, ssk = 0.0f;
 #pragma unroll
@@ -357,23 +376,11 @@ __global__ __launch_bounds__(256) void qk_rmsnorm_rope_split128_kernel(
   auto finish = [&](const uint4* xa, const uint4* xb, float r, const void* w, uint16_t* yr) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int p = i * 64 + lane, h = p >> 3, k = p & 7;
-      const int col = h * 128 + k * 8;
-      float a[8], b[8], o0[8], o1[8];
+      float a[8], b[8];
       e_unpack8<H>(xa[i], a);
       e_unpack8<H>(xb[i], b);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-#pragma clang fp contract(off)
-        const float n0 = a[j] * r * (load_w<WT>(w, col + j) + weight_offset);
-        const float n1 = b[j] * r * (load_w<WT>(w, col + 64 + j) + weight_offset);
-        const float fc = n0 * c[i][j], ss2 = n1 * sn[i][j];  // first * c, second * s
-        const float fs = n0 * sn[i][j], sc = n1 * c[i][j];   // first * s, second * c
-        o0[j] = fc - ss2;
-        o1[j] = fs + sc;
-      }
-      *reinterpret_cast<uint4*>(yr + col) = e_pack8<H>(o0);
-      *reinterpret_cast<uint4*>(yr + col + 64) = e_pack8<H>(o1);
+      split_rotate<H, HALF, WT>(a, b, r, w, wvec, weight_offset, c[i], sn[i], yr,
+                                SplitChunk<HALF>(i * 64 + lane).col);
     }
   };
   finish(qa, qb, rq, wq, yq + row * ldyq);
@@ -407,30 +414,77 @@ __global__ __launch_bounds__(256) void rmsnorm_generic(
 // ----------------------------------------------------------------------------------------------
 // Elementwise row ops with fp32 modulation rows.
 
-template <bool H>
+// V columns per thread: 8 where rows, strides and addresses allow 16-byte accesses, else 1.
+template <bool H, int V>
+__device__ __forceinline__ void load_v(const uint16_t* p, float* v) {
+  if constexpr (V == 8) e_unpack8<H>(*reinterpret_cast<const uint4*>(p), v);
+  else v[0] = e2f<H>(*p);
+}
+template <bool H, int V>
+__device__ __forceinline__ void store_v(uint16_t* p, const float* v) {
+  if constexpr (V == 8) *reinterpret_cast<uint4*>(p) = e_pack8<H>(v);
+  else *p = f2e<H>(v[0]);
+}
+template <int V>
+__device__ __forceinline__ void load_mod(const float* p, float* v) {
+  if constexpr (V == 8) load_f8(p, v);
+  else v[0] = *p;
+}
+
+template <bool H, int V>
 __global__ __launch_bounds__(256) void modulate_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy,
     int64_t rows, int64_t dim, const float* __restrict__ shift, const float* __restrict__ scale,
     int64_t mod_div, int64_t mod_stride) {
-  const int64_t per_row = dim;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t per_row = dim / V;
   if (idx >= rows * per_row) return;
-  const int64_t r = idx / per_row, c = idx - r * per_row;
+  const int64_t r = idx / per_row, c = (idx - r * per_row) * V;
   const int64_t m = (r / mod_div) * mod_stride + c;
-  y[r * ldy + c] = f2e<H>(e2f<H>(x[r * ldx + c]) * (1.0f + scale[m]) + shift[m]);
+  float v[V], sc[V], sh[V];
+  load_v<H, V>(x + r * ldx + c, v);
+  load_mod<V>(scale + m, sc);
+  load_mod<V>(shift + m, sh);
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = v[j] * (1.0f + sc[j]) + sh[j];
+  store_v<H, V>(y + r * ldy + c, v);
 }
 
-template <bool H>
+template <bool H, int V>
 __global__ __launch_bounds__(256) void gated_residual_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ r, int64_t ldr,
     uint16_t* __restrict__ y, int64_t ldy, int64_t rows, int64_t dim,
     const float* __restrict__ gate, int64_t gate_div, int64_t gate_stride) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= rows * dim) return;
-  const int64_t row = idx / dim, c = idx - row * dim;
-  const float g = gate[(row / gate_div) * gate_stride + c];
-  const float base = x ? e2f<H>(x[row * ldx + c]) : 0.0f;
-  y[row * ldy + c] = f2e<H>(base + e2f<H>(r[row * ldr + c]) * g);
+  const int64_t per_row = dim / V;
+  if (idx >= rows * per_row) return;
+  const int64_t row = idx / per_row, c = (idx - row * per_row) * V;
+  float g[V], base[V], v[V];
+  load_mod<V>(gate + (row / gate_div) * gate_stride + c, g);
+  load_v<H, V>(r + row * ldr + c, v);
+#pragma unroll
+  for (int j = 0; j < V; ++j) base[j] = 0.0f;
+  if (x) load_v<H, V>(x + row * ldx + c, base);
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = base[j] + v[j] * g[j];
+  store_v<H, V>(y + row * ldy + c, v);
+}
+
+// out[r][i][c] = fp32(projected[r][i * dim + c]) + fp32(table[i][c]) for the six modulation rows of a
+// block; the scale rows (0 and 3) with the zero-centred norm weight that follows folded in:
+// (1 + scale) (1 + w) - 1, each operation rounded in fp32.
+template <int PT, int TT>
+__global__ __launch_bounds__(256) void six_way_modulation_kernel(
+    const void* __restrict__ projected, int64_t ldp, const void* __restrict__ table, const float* __restrict__ w1,
+    const float* __restrict__ w2, float* __restrict__ out, int64_t total, int dim) {
+#pragma clang fp contract(off)
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= total) return;
+  const int64_t r = idx / (6 * dim);
+  const int e = (int)(idx - r * (6 * dim)), i = e / dim, c = e - i * dim;
+  float v = load_w<PT>(projected, r * ldp + e) + load_w<TT>(table, e);
+  if (i == 0 || i == 3) v = (1.0f + v) * (1.0f + (i == 0 ? w1 : w2)[c]) - 1.0f;
+  out[idx] = v;
 }
 
 template <bool H, int VPL, int KIND, bool XF32>
@@ -455,7 +509,12 @@ int dispatch_adaln(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t row
     switch (dim / 512) {
       case 1: return launch_adaln<H, 1, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
       case 2: return launch_adaln<H, 2, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
+      case 3: return launch_adaln<H, 3, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
       case 4: return launch_adaln<H, 4, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
+      case 5: return launch_adaln<H, 5, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
+      case 6: return launch_adaln<H, 6, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
+      case 10: return launch_adaln<H, 10, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
+      case 12: return launch_adaln<H, 12, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
       default: return launch_adaln<H, 8, KIND, XF32>(x, ldx, y, ldy, rows, shift, scale, mod_div, mod_stride, eps, s);
     }
   }
@@ -530,8 +589,9 @@ int adaln_norm(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, i
   KX_REQUIRE(kind == KX_NORM_RMS || kind == KX_NORM_LAYER, "%s: bad kind", name);
   if (rows == 0) return KX_OK;
   const int64_t vpl = dim / 512;
-  const bool vec = dim % 512 == 0 && (vpl == 1 || vpl == 2 || vpl == 4 || vpl == 8) &&
-                   ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y) &&
+  // widths of 512 .. 3072, 4096, 5120 and 6144 keep their rows in registers (3072 wide, 2305 rows: 42 us in
+  // the strided loop, 8 in registers)
+  const bool vec = dim % 512 == 0 && (vpl <= 6 || vpl == 8 || vpl == 10 || vpl == 12) && ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y) &&
                    (!shift || (aligned16(shift) && aligned16(scale) && mod_stride % 4 == 0));
   if (xf32)
     return kind == KX_NORM_RMS
@@ -564,12 +624,19 @@ int rmsnorm_rope(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
   else if (rope_kind == KX_ROPE_PAIR)
     rope_ok = 512 % head_dim == 0 && head_dim >= 8;
   const bool align_ok = ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y);
-  if (shape_ok && align_ok && rope_kind == KX_ROPE_SPLIT && norm_width == dim && head_dim == 128 &&
-      vpl >= 2 && table_ld % 4 == 0 && table_hs % 4 == 0 && aligned16(cos) && aligned16(sin)) {
+  // 64-wide heads: 5376 x 2048 rows 71 -> 22 us against rmsnorm_rope_kernel, whose rotation takes
+  // lane exchanges and 4-byte table and 2-byte weight loads
+  if (shape_ok && align_ok && rope_kind == KX_ROPE_SPLIT && norm_width == dim &&
+      (head_dim == 128 || head_dim == 64) && vpl >= 2 && table_ld % 4 == 0 && table_hs % 4 == 0 && aligned16(cos) &&
+      aligned16(sin)) {
     const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
-#define KX_RS(V)                                                                                          \
-  rmsnorm_rope_split128_kernel<H, V, WT><<<grid, 256, 0, s>>>((const uint16_t*)x, ldx, (uint16_t*)y, ldy, rows, \
-      w, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);                        \
+    const bool wvec = aligned16(w);
+#define KX_RSH(V, HALF)                                                                                      \
+  rmsnorm_rope_split_kernel<H, HALF, V, WT><<<grid, 256, 0, s>>>((const uint16_t*)x, ldx, (uint16_t*)y, ldy, rows, \
+      w, wvec, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);
+#define KX_RS(V)                              \
+  if (head_dim == 128) { KX_RSH(V, 64) }      \
+  else { KX_RSH(V, 32) }                      \
   return check_launch(name);
     switch (vpl) {
       case 2: KX_RS(2)
@@ -577,6 +644,7 @@ int rmsnorm_rope(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
       default: KX_RS(8)
     }
 #undef KX_RS
+#undef KX_RSH
   }
   if (shape_ok && rope_ok && align_ok) {
 #define KX_RR(V)                                                                                       \
@@ -629,12 +697,11 @@ int rmsnorm_rope_checked(const void* x, int64_t ldx, void* y, int64_t ldy, int64
 #undef KX_RN
 }
 
-template <bool H>
-int qk_rmsnorm_rope(const void* xq, int64_t ldq, const void* xk, int64_t ldk, void* yq, int64_t ldyq, void* yk,
+template <bool H, int HALF>
+int qk_rmsnorm_rope(const char* name, const void* xq, int64_t ldq, const void* xk, int64_t ldk, void* yq, int64_t ldyq, void* yk,
                     int64_t ldyk, int64_t rows, int64_t dim, const void* wq, const void* wk, int w_dtype, float eps,
                     float weight_offset, const float* cos, const float* sin, int64_t table_ld, int64_t table_hs,
                     int64_t tokens, int table_batched, hipStream_t s) {
-  const char* name = ename<H>("kx_qk_rmsnorm_rope_bf16", "kx_qk_rmsnorm_rope_f16");
   KX_REQUIRE(xq && xk && yq && yk && wq && wk && cos && sin, "%s: null tensor", name);
   KX_REQUIRE(rows >= 0 && dim > 0 && ldq >= dim && ldk >= dim && ldyq >= dim && ldyk >= dim, "%s: bad shape", name);
   KX_REQUIRE(w_dtype == KX_F32 || w_dtype == KX_BF16 || w_dtype == KX_F16, "%s: bad weight dtype", name);
@@ -645,13 +712,15 @@ int qk_rmsnorm_rope(const void* xq, int64_t ldq, const void* xk, int64_t ldk, vo
                   aligned16(yk) && table_ld % 4 == 0 && table_hs % 4 == 0 && aligned16(cos) && aligned16(sin);
   if (!ok)
     return set_error(KX_ERR_UNSUPPORTED,
-                     "%s: needs dim in {1024, 2048, 4096}, 128-wide heads and 16-byte aligned rows and tables", name);
+                     "%s: needs dim in {1024, 2048, 4096}, %d-wide heads and 16-byte aligned rows and tables", name,
+                     2 * HALF);
   if (rows == 0) return KX_OK;
   const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
+  const bool wvec = aligned16(wq) && aligned16(wk);
 #define KX_QK(V, WT)                                                                                        \
-  qk_rmsnorm_rope_split128_kernel<H, V, WT><<<grid, 256, 0, s>>>(                                            \
+  qk_rmsnorm_rope_split_kernel<H, HALF, V, WT><<<grid, 256, 0, s>>>(                                         \
       (const uint16_t*)xq, ldq, (const uint16_t*)xk, ldk, (uint16_t*)yq, ldyq, (uint16_t*)yk, ldyk, rows, wq, wk, \
-      eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);                              \
+      wvec, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);                        \
   return check_launch(name);
 #define KX_QKW(V)                          \
   switch (w_dtype) {                       \
@@ -677,8 +746,14 @@ int modulate(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, int
              name);
   const int64_t total = rows * dim;
   if (total == 0) return KX_OK;
-  modulate_kernel<H><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(
-      (const uint16_t*)x, ldx, (uint16_t*)y, ldy, rows, dim, shift, scale, mod_div, mod_stride);
+  const bool vec = dim % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 && mod_stride % 4 == 0 && aligned16(x) && aligned16(y) &&
+                   aligned16(shift) && aligned16(scale);
+  if (vec)
+    modulate_kernel<H, 8><<<(unsigned)((total / 8 + 255) / 256), 256, 0, s>>>(
+        (const uint16_t*)x, ldx, (uint16_t*)y, ldy, rows, dim, shift, scale, mod_div, mod_stride);
+  else
+    modulate_kernel<H, 1><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(
+        (const uint16_t*)x, ldx, (uint16_t*)y, ldy, rows, dim, shift, scale, mod_div, mod_stride);
   return check_launch(name);
 }
 
@@ -692,8 +767,14 @@ int gated_residual(const void* x, int64_t ldx, const void* r, int64_t ldr, void*
              "%s: bad shape", name);
   const int64_t total = rows * dim;
   if (total == 0) return KX_OK;
-  gated_residual_kernel<H><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(
-      (const uint16_t*)x, ldx, (const uint16_t*)r, ldr, (uint16_t*)y, ldy, rows, dim, gate, gate_div, gate_stride);
+  const bool vec = dim % 8 == 0 && ldr % 8 == 0 && ldy % 8 == 0 && gate_stride % 4 == 0 && aligned16(r) && aligned16(y) &&
+                   aligned16(gate) && (!x || (ldx % 8 == 0 && aligned16(x)));
+  if (vec)  // 2305 x 3072: 18 us one element per thread, 12 in vectors
+    gated_residual_kernel<H, 8><<<(unsigned)((total / 8 + 255) / 256), 256, 0, s>>>(
+        (const uint16_t*)x, ldx, (const uint16_t*)r, ldr, (uint16_t*)y, ldy, rows, dim, gate, gate_div, gate_stride);
+  else
+    gated_residual_kernel<H, 1><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(
+        (const uint16_t*)x, ldx, (const uint16_t*)r, ldr, (uint16_t*)y, ldy, rows, dim, gate, gate_div, gate_stride);
   return check_launch(name);
 }
 
@@ -724,9 +805,19 @@ using namespace kx;
                                              float weight_offset, const float* cos, const float* sin,             \
                                              int64_t table_ld, int64_t table_hs, int64_t tokens,                  \
                                              int table_batched, kx_stream_t stream) {                             \
-    return qk_rmsnorm_rope<H>(xq, ldq, xk, ldk, yq, ldyq, yk, ldyk, rows, dim, wq, wk, w_dtype, eps,              \
-                              weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched,                 \
-                              (hipStream_t)stream);                                                               \
+    return qk_rmsnorm_rope<H, 64>("kx_qk_rmsnorm_rope_" #SUFFIX, xq, ldq, xk, ldk, yq, ldyq, yk, ldyk, rows, dim, \
+                                  wq, wk, w_dtype, eps, weight_offset, cos, sin, table_ld, table_hs, tokens,      \
+                                  table_batched, (hipStream_t)stream);                                            \
+  }                                                                                                               \
+  extern "C" int kx_qk_rmsnorm_rope_h64_##SUFFIX(const void* xq, int64_t ldq, const void* xk, int64_t ldk,       \
+                                                 void* yq, int64_t ldyq, void* yk, int64_t ldyk, int64_t rows,    \
+                                                 int64_t dim, const void* wq, const void* wk, int w_dtype,        \
+                                                 float eps, float weight_offset, const float* cos,                \
+                                                 const float* sin, int64_t table_ld, int64_t table_hs,            \
+                                                 int64_t tokens, int table_batched, kx_stream_t stream) {         \
+    return qk_rmsnorm_rope<H, 32>("kx_qk_rmsnorm_rope_h64_" #SUFFIX, xq, ldq, xk, ldk, yq, ldyq, yk, ldyk, rows, \
+                                  dim, wq, wk, w_dtype, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, \
+                                  table_batched, (hipStream_t)stream);                                            \
   }                                                                                                               \
   extern "C" int kx_modulate_##SUFFIX(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,            \
                                       int64_t dim, const float* shift, const float* scale, int64_t mod_div,       \
@@ -742,3 +833,33 @@ using namespace kx;
 
 KX_NORM_ENTRY(bf16, false)
 KX_NORM_ENTRY(f16, true)
+
+extern "C" int kx_six_way_modulation_f32(const void* projected, int p_dtype, int64_t ldp, const void* table,
+                                         int t_dtype, const float* w1, const float* w2, float* out, int64_t rows,
+                                         int64_t dim, kx_stream_t stream) {
+  const char* name = "kx_six_way_modulation_f32";
+  KX_REQUIRE(projected && table && w1 && w2 && out, "%s: null tensor", name);
+  KX_REQUIRE(rows >= 0 && dim > 0 && dim < (1 << 28) && ldp >= 6 * dim, "%s: bad shape", name);
+  KX_REQUIRE(p_dtype >= KX_F32 && p_dtype <= KX_F16 && t_dtype >= KX_F32 && t_dtype <= KX_F16,
+             "%s: dtypes must be KX_F32, KX_BF16 or KX_F16", name);
+  const int64_t total = rows * 6 * dim;
+  KX_REQUIRE(total / 256 < (1ll << 31), "%s: too many elements", name);
+  if (total == 0) return KX_OK;
+  const unsigned grid = (unsigned)((total + 255) / 256);
+  hipStream_t s = (hipStream_t)stream;
+#define KX_SIX(PT, TT) six_way_modulation_kernel<PT, TT><<<grid, 256, 0, s>>>(projected, ldp, table, w1, w2, out, total, (int)dim)
+#define KX_SIX_T(PT)                              \
+  switch (t_dtype) {                              \
+    case KX_BF16: KX_SIX(PT, KX_BF16); break;     \
+    case KX_F16: KX_SIX(PT, KX_F16); break;       \
+    default: KX_SIX(PT, KX_F32);                  \
+  }
+  switch (p_dtype) {
+    case KX_BF16: KX_SIX_T(KX_BF16) break;
+    case KX_F16: KX_SIX_T(KX_F16) break;
+    default: KX_SIX_T(KX_F32)
+  }
+#undef KX_SIX_T
+#undef KX_SIX
+  return check_launch(name);
+}

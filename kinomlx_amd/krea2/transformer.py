@@ -266,14 +266,19 @@ class Krea2SwiGLU:
         return self.down(hidden, residual=residual, gate=residual_gate, out_dtype=out_dtype)
 
 
-def split_six_way_modulation(projected: torch.Tensor, scale_shift_table: torch.Tensor) -> tuple[torch.Tensor, ...]:
-    """Add one block's ``(6, hidden)`` table and return the official chunk order
-    (``model.py:288-307``): prescale, preshift, pregate, postscale, postshift, postgate."""
+def _check_six_way(projected: torch.Tensor, scale_shift_table: torch.Tensor) -> None:
     if scale_shift_table.dim() != 2 or scale_shift_table.shape[0] != 6:
         raise ValueError("Krea block modulation table must have shape [6, hidden]")
     hidden_size = scale_shift_table.shape[1]
     if projected.shape[-1] != 6 * hidden_size:
         raise ValueError("Krea projected modulation width must be six times hidden size")
+
+
+def split_six_way_modulation(projected: torch.Tensor, scale_shift_table: torch.Tensor) -> tuple[torch.Tensor, ...]:
+    """Add one block's ``(6, hidden)`` table and return the official chunk order
+    (``model.py:288-307``): prescale, preshift, pregate, postscale, postshift, postgate."""
+    _check_six_way(projected, scale_shift_table)
+    hidden_size = scale_shift_table.shape[1]
     modulation = projected.reshape(*projected.shape[:-1], 6, hidden_size) + scale_shift_table
     return tuple(modulation[..., i, :] for i in range(6))
 
@@ -308,25 +313,26 @@ class Krea2TransformerBlock:
         self.attn.fuse_projections()
         self.ff.fuse_projections()
 
-    def _modulated(self, value: torch.Tensor, norm: Krea2RMSNorm, scale: torch.Tensor,
-                   shift: torch.Tensor) -> torch.Tensor:
-        """``(1 + scale) * norm(x) + shift`` in one FP32 pass: the zero-centred weight is folded
-        into the scale, ``(1 + scale)(1 + w) = 1 + scale'``."""
-        if norm.weight is None:
+    def _modulation(self, projected: torch.Tensor) -> tuple[torch.Tensor, ...]:
+        """``split_six_way_modulation`` in one pass, each scale with the zero-centred norm weight it
+        multiplies folded in: ``(1 + scale)(1 + w) = 1 + scale'``, so that the modulated norm is one
+        AdaLN pass."""
+        table = self.scale_shift_table
+        if self.norm1.weight is None or self.norm2.weight is None:
             raise ValueError("Krea RMSNorm weight is not loaded")
-        scale_eff = (1.0 + scale.float()) * (1.0 + norm.weight.float()) - 1.0
-        return adaln(value, scale_eff, shift.float().expand_as(scale_eff), norm.eps)
+        _check_six_way(projected, table)
+        modulation = _lib.six_way_modulation(projected, table, self.norm1.weight, self.norm2.weight)
+        return tuple(modulation[..., i, :] for i in range(6))
 
     def __call__(self, hidden_states: torch.Tensor, *, time_modulation: torch.Tensor,
                  rotary: tuple[torch.Tensor, torch.Tensor], attention_mask: torch.Tensor | None,
                  reference_attention=None) -> torch.Tensor:
         if hidden_states.dtype != torch.bfloat16:
             raise ValueError("Krea2TransformerBlock takes bfloat16 hidden states on MI355X")
-        prescale, preshift, pregate, postscale, postshift, postgate = split_six_way_modulation(
-            time_modulation, self.scale_shift_table)
-        attention_input = self._modulated(hidden_states, self.norm1, prescale, preshift)
+        prescale, preshift, pregate, postscale, postshift, postgate = self._modulation(time_modulation)
+        attention_input = adaln(hidden_states, prescale, preshift, self.norm1.eps)
         h1 = self.attn(attention_input, attention_mask=attention_mask, rotary=rotary,
                        reference_attention=reference_attention, residual=hidden_states, gate=pregate,
                        out_dtype=torch.float32)
-        feed_forward_input = self._modulated(h1, self.norm2, postscale, postshift)
+        feed_forward_input = adaln(h1, postscale, postshift, self.norm2.eps)
         return self.ff(feed_forward_input, residual=h1, residual_gate=postgate, out_dtype=hidden_states.dtype)

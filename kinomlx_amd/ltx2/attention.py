@@ -107,7 +107,7 @@ def norm_rope_qk(q_raw: torch.Tensor, k_raw: torch.Tensor, q_norm: RMSNorm, k_no
     batch, tokens, dim = q_raw.shape
     head_dim = dim // heads
     cos, sin = pe
-    if (head_dim != 128 or q_norm.weight is None or k_norm.weight is None or q_norm.eps != k_norm.eps
+    if (head_dim not in (64, 128) or q_norm.weight is None or k_norm.weight is None or q_norm.eps != k_norm.eps
             or q_norm.weight.dtype != k_norm.weight.dtype or not (cos.dim() == 4 and cos.shape[1] == heads
             and cos.shape[2] == tokens and cos.shape[3] * 2 == head_dim and cos.shape[0] in (1, batch)
             and cos.dtype == torch.float32 and cos.shape == sin.shape)):
@@ -119,7 +119,7 @@ def norm_rope_qk(q_raw: torch.Tensor, k_raw: torch.Tensor, q_norm: RMSNorm, k_no
     cos_tm, sin_tm = split_rope.token_major(cos), split_rope.token_major(sin)
     if not _lib.launch_qk_rmsnorm_rope(q_raw, k_raw, q, k, q_norm.weight, k_norm.weight, q_norm.eps, cos=cos_tm,
                                        sin=sin_tm, table_ld=heads * head_dim // 2, table_hs=head_dim // 2,
-                                       tokens=tokens, table_batched=cos.shape[0] > 1):
+                                       tokens=tokens, table_batched=cos.shape[0] > 1, head_dim=head_dim):
         return None
     return q, k
 
