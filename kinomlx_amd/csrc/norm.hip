@@ -139,18 +139,6 @@ __device__ __forceinline__ float load_w(const void* w, int64_t i) {
   else return reinterpret_cast<const float*>(w)[i];
 }
 
-// Eight consecutive weights from column i (a multiple of 8): vector loads where the weight is 16-byte
-// aligned (vec), the same values one by one where it is a view at another offset.
-template <int WT>
-__device__ __forceinline__ void load_w8(const void* w, int64_t i, bool vec, float* v) {
-  if (vec) {
-    load8<WT == KX_F16, WT == KX_F32>(w, i, v);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = load_w<WT>(w, i + j);
-  }
-}
-
 template <bool H, int VPL, int G, int ROPE, int WT>
 __global__ __launch_bounds__(256) void rmsnorm_rope_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy,
@@ -192,10 +180,9 @@ __global__ __launch_bounds__(256) void rmsnorm_rope_kernel(
   for (int i = 0; i < VPL; ++i) {
     const int col = (i * 64 + lane) * 8;
     const int wcol = (G == 0) ? col : (col % norm_width);
-    float wv[8];
-    load_w8<WT>(w, wcol, (reinterpret_cast<uintptr_t>(w) & 15) == 0, wv);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * inv[i] * (wv[j] + weight_offset);
+    for (int j = 0; j < 8; ++j)
+      v[i][j] = v[i][j] * inv[i] * (load_w<WT>(w, wcol + j) + weight_offset);
   }
   uint16_t* yr = y + row * ldy;
   if (ROPE == KX_ROPE_NONE) {
@@ -275,17 +262,15 @@ __device__ __forceinline__ void load_f8(const float* p, float* v) {
 }
 // One chunk pair normalized by r, weighted and rotated, to yr + col and yr + col + HALF.
 template <bool H, int HALF, int WT>
-__device__ __forceinline__ void split_rotate(const float* a, const float* b, float r, const void* w, bool wvec,
+__device__ __forceinline__ void split_rotate(const float* a, const float* b, float r, const void* w,
                                              float weight_offset, const float* c, const float* sn, uint16_t* yr,
                                              int col) {
-  float w0[8], w1[8], o0[8], o1[8];
-  load_w8<WT>(w, col, wvec, w0);
-  load_w8<WT>(w, col + HALF, wvec, w1);
+  float o0[8], o1[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
 #pragma clang fp contract(off)
-    const float n0 = a[j] * r * (w0[j] + weight_offset);
-    const float n1 = b[j] * r * (w1[j] + weight_offset);
+    const float n0 = a[j] * r * (load_w<WT>(w, col + j) + weight_offset);
+    const float n1 = b[j] * r * (load_w<WT>(w, col + HALF + j) + weight_offset);
     const float fc = n0 * c[j], ss2 = n1 * sn[j];  // first * c, second * s
     const float fs = n0 * sn[j], sc = n1 * c[j];   // first * s, second * c
     o0[j] = fc - ss2;
@@ -298,7 +283,7 @@ __device__ __forceinline__ void split_rotate(const float* a, const float* b, flo
 template <bool H, int HALF, int VPL, int WT>
 __global__ __launch_bounds__(256) void rmsnorm_rope_split_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy,
-    int64_t rows, const void* __restrict__ w, bool wvec, float eps, float weight_offset,
+    int64_t rows, const void* __restrict__ w, float eps, float weight_offset,
     const float* __restrict__ cosp, const float* __restrict__ sinp, int64_t table_ld,
     int64_t table_hs, int64_t tokens, int table_batched) {
   constexpr int DIM = VPL * 512;
@@ -325,7 +310,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rope_split_kernel(
   const float r = rsqrtf(wave_sum<64>(ss) * (1.0f / DIM) + eps);
 #pragma unroll
   for (int i = 0; i < NP; ++i)
-    split_rotate<H, HALF, WT>(a[i], b[i], r, w, wvec, weight_offset, c[i], sn[i], y + row * ldy,
+    split_rotate<H, HALF, WT>(a[i], b[i], r, w, weight_offset, c[i], sn[i], y + row * ldy,
                               SplitChunk<HALF>(i * 64 + lane).col);
 }
 
@@ -337,7 +322,7 @@ template <bool H, int HALF, int VPL, int WT>
 __global__ __launch_bounds__(256) void qk_rmsnorm_rope_split_kernel(
     const uint16_t* __restrict__ xq, int64_t ldq, const uint16_t* __restrict__ xk, int64_t ldk,
     uint16_t* __restrict__ yq, int64_t ldyq, uint16_t* __restrict__ yk, int64_t ldyk, int64_t rows,
-    const void* __restrict__ wq, const void* __restrict__ wk, bool wvec, float eps, float weight_offset,
+    const void* __restrict__ wq, const void* __restrict__ wk, float eps, float weight_offset,
     const float* __restrict__ cosp, const float* __restrict__ sinp, int64_t table_ld,
     int64_t table_hs, int64_t tokens, int table_batched) {
   constexpr int DIM = VPL * 512;
@@ -379,7 +364,7 @@ __global__ __launch_bounds__(256) void qk_rmsnorm_rope_split_kernel(
       float a[8], b[8];
       e_unpack8<H>(xa[i], a);
       e_unpack8<H>(xb[i], b);
-      split_rotate<H, HALF, WT>(a, b, r, w, wvec, weight_offset, c[i], sn[i], yr,
+      split_rotate<H, HALF, WT>(a, b, r, w, weight_offset, c[i], sn[i], yr,
                                 SplitChunk<HALF>(i * 64 + lane).col);
     }
   };
@@ -589,8 +574,8 @@ int adaln_norm(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, i
   KX_REQUIRE(kind == KX_NORM_RMS || kind == KX_NORM_LAYER, "%s: bad kind", name);
   if (rows == 0) return KX_OK;
   const int64_t vpl = dim / 512;
-  // widths of 512 .. 3072, 4096, 5120 and 6144 keep their rows in registers (3072 wide, 2305 rows: 42 us in
-  // the strided loop, 8 in registers)
+  // widths of 512 .. 3072, 4096, 5120 and 6144 keep their rows in registers (3072 wide, 2305 rows: 28 us in
+  // the strided loop, 12 in registers)
   const bool vec = dim % 512 == 0 && (vpl <= 6 || vpl == 8 || vpl == 10 || vpl == 12) && ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y) &&
                    (!shift || (aligned16(shift) && aligned16(scale) && mod_stride % 4 == 0));
   if (xf32)
@@ -624,16 +609,15 @@ int rmsnorm_rope(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
   else if (rope_kind == KX_ROPE_PAIR)
     rope_ok = 512 % head_dim == 0 && head_dim >= 8;
   const bool align_ok = ldx % 8 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y);
-  // 64-wide heads: 5376 x 2048 rows 71 -> 22 us against rmsnorm_rope_kernel, whose rotation takes
-  // lane exchanges and 4-byte table and 2-byte weight loads
+  // 64-wide heads: 5376 x 2048 rows 28 -> 13 us (36 -> 26 out of HBM) against rmsnorm_rope_kernel, whose
+  // rotation takes lane exchanges and 4-byte table loads
   if (shape_ok && align_ok && rope_kind == KX_ROPE_SPLIT && norm_width == dim &&
       (head_dim == 128 || head_dim == 64) && vpl >= 2 && table_ld % 4 == 0 && table_hs % 4 == 0 && aligned16(cos) &&
       aligned16(sin)) {
     const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
-    const bool wvec = aligned16(w);
 #define KX_RSH(V, HALF)                                                                                      \
   rmsnorm_rope_split_kernel<H, HALF, V, WT><<<grid, 256, 0, s>>>((const uint16_t*)x, ldx, (uint16_t*)y, ldy, rows, \
-      w, wvec, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);
+      w, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);
 #define KX_RS(V)                              \
   if (head_dim == 128) { KX_RSH(V, 64) }      \
   else { KX_RSH(V, 32) }                      \
@@ -716,11 +700,10 @@ int qk_rmsnorm_rope(const char* name, const void* xq, int64_t ldq, const void* x
                      2 * HALF);
   if (rows == 0) return KX_OK;
   const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
-  const bool wvec = aligned16(wq) && aligned16(wk);
 #define KX_QK(V, WT)                                                                                        \
   qk_rmsnorm_rope_split_kernel<H, HALF, V, WT><<<grid, 256, 0, s>>>(                                         \
       (const uint16_t*)xq, ldq, (const uint16_t*)xk, ldk, (uint16_t*)yq, ldyq, (uint16_t*)yk, ldyk, rows, wq, wk, \
-      wvec, eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);                        \
+      eps, weight_offset, cos, sin, table_ld, table_hs, tokens, table_batched);                              \
   return check_launch(name);
 #define KX_QKW(V)                          \
   switch (w_dtype) {                       \
@@ -769,7 +752,7 @@ int gated_residual(const void* x, int64_t ldx, const void* r, int64_t ldr, void*
   if (total == 0) return KX_OK;
   const bool vec = dim % 8 == 0 && ldr % 8 == 0 && ldy % 8 == 0 && gate_stride % 4 == 0 && aligned16(r) && aligned16(y) &&
                    aligned16(gate) && (!x || (ldx % 8 == 0 && aligned16(x)));
-  if (vec)  // 2305 x 3072: 18 us one element per thread, 12 in vectors
+  if (vec)  // 2305 x 3072: 17 us one element per thread, 12 in vectors
     gated_residual_kernel<H, 8><<<(unsigned)((total / 8 + 255) / 256), 256, 0, s>>>(
         (const uint16_t*)x, ldx, (const uint16_t*)r, ldr, (uint16_t*)y, ldy, rows, dim, gate, gate_div, gate_stride);
   else

@@ -46,7 +46,7 @@ def test_adaln_widths(device, dim, dtype, kind):
 @pytest.mark.parametrize("dim", [1024, 2048, 4096])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_split_rope_of_64_wide_heads(device, dim, dtype, offset):
-    """Norm + RoPE of one tensor against the oracle, with a 16-byte aligned weight and one that
+    """Norm + RoPE of one tensor against the oracle, with an aligned weight and one that
     starts an element later; Q and K in one pass give the same bits as one at a time."""
     heads, tokens = dim // 64, 7
     q, k = (_t((2, tokens, dim), s).to(device, dtype) for s in (1, 2))
