@@ -44,6 +44,9 @@ EPI_GATED_RESIDUAL = 1 << 8
 EPI_RESID_F32 = 1 << 9
 EPI_OUT_F32 = 1 << 10
 
+# A dtype argument of the native launch path; None: the function's default
+DTYPE_CODES = {None: -1, torch.float32: KX_F32, torch.bfloat16: KX_BF16, torch.float16: KX_F16}
+
 _P = ctypes.c_void_p
 _I64 = ctypes.c_int64
 _I = ctypes.c_int
@@ -169,6 +172,32 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native launch path (``_host.so``), bound to the loaded library; None while a ``LaunchTimer``
+    is installed (its events bracket each entry point on the Python path). Its functions return None
+    for a call they leave to the Python code."""
+    if _timer is not None:
+        return None
+    return _host if _host is not None else _bind_host()
+
+
+def _bind_host():
+    global _host
+    lib = load()
+    try:
+        from . import _host as module
+    except ImportError as exc:
+        raise RuntimeError(f"the native launch path is not built ({exc}); run `python -m kinomlx_amd.csrc.build`") from exc
+    names = [*SIGNATURES, "kx_last_error"]
+    module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names}, KernelError,
+                gemm_plan, lambda batch, tq, tk, heads: (0, attention_splits(batch, tq, tk, heads)))
+    _host = module
+    return module
+
+
 def available() -> bool:
     """Whether the library is built and a GPU is visible to torch."""
     return LIBRARY_PATH.exists() and torch.cuda.is_available()
@@ -219,7 +248,9 @@ def _call(name: str, *args, unsupported_ok: bool = False) -> int:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream, as ``torch.cuda.current_stream().cuda_stream`` (whose Python
+    wrapper takes 5 us; this takes 0.2)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -546,6 +577,11 @@ def launch_gemm_columns(a, w, out, *, bias=None, q_end: int = 0, k_end: int = 0,
     as in ``launch_gemm_qknorm_rope`` (``k_end`` 0: none), and the columns from ``swiglu_begin`` on,
     ``[gate | up]``, written as ``silu(gate) * up`` to ``swiglu_out`` (None: no such columns). ``out``
     holds the columns before ``swiglu_begin`` (None when there are none)."""
+    if a.is_cuda and table_hs == 0 and (native := host()) is not None:
+        begin = int(w.shape[0]) if swiglu_out is None else swiglu_begin
+        if native.columns(a, w, bias, out, q_end, k_end, head_dim, norm_q, norm_k, eps, weight_offset, cos, sin,
+                          table_ld, table_rows, table_bs, begin, swiglu_out, _stream()) is not None:
+            return
     _check_gpu("gemm_columns", a, w, out, bias, norm_q, norm_k, cos, sin, swiglu_out)
     m, k, lda = _rows(a, "projection input")
     n, kw, ldw = _rows(w, "projection weight")
@@ -633,6 +669,13 @@ def splitk_splits(m: int, n: int, k: int) -> int:
     if load().kx_gemm_splits(m, n, k, ctypes.addressof(out)) != KX_OK:
         raise KernelError(f"kx_gemm_splits: bad shape ({m}, {n}, {k})")
     return out.value
+
+
+def gemm_plan(m: int, n: int, k: int) -> tuple[int, int]:
+    """``(rows, splits)`` of a dense product: with ``rows`` > 0 the last ``m - rows`` rows run as
+    ``splits`` K slices before the first rows (``tail_split``), else the whole product as ``splits``."""
+    tail = tail_split(m, n, k)
+    return tail if tail is not None else (0, splitk_splits(m, n, k))
 
 
 def launch_qgemm(a, words, scales, biases, out, *, n, k, group_size, bits, bias=None,
@@ -794,6 +837,10 @@ def table_add(table: torch.Tensor, ts: torch.Tensor | None, round_to: torch.dtyp
     ``(rows, D)`` (fp32, bf16 or fp16), ``ts`` ``(B, T, rows, D)`` with a contiguous last axis (other
     strides may be 0 to broadcast), or ``None`` (the table alone, as ``(1, 1, rows, D)``). With
     ``round_to`` bf16 or fp16 every sum is rounded to that type (and kept as fp32)."""
+    if table.is_cuda and (native := host()) is not None:
+        code = DTYPE_CODES.get(round_to, -1)
+        if code >= 0 and (out := native.table_add(table, ts, code, _stream())) is not None:
+            return out
     _check_gpu("table_add", table, ts)
     if table.dim() != 2 or table.stride(-1) != 1 or (table.shape[0] > 1 and table.stride(0) != table.shape[1]):
         raise ValueError("table_add: table must be a contiguous (rows, dim) tensor")

@@ -150,6 +150,13 @@ def fused_linear(
     residual stream can be carried in fp32 between blocks' branches so that it is rounded once, not
     once per add.
     """
+    if value.is_cuda and (native := _lib.host()) is not None:
+        code = _lib.DTYPE_CODES.get(out_dtype)
+        if code is not None:
+            result = native.linear(value, _weight(weight), bias, ACTIVATIONS[activation], residual, gate, out, code,
+                                   _lib._stream())
+            if result is not None:
+                return result
     w = _as_out_in(weight, True)
     dtype = value.dtype
     if dtype not in _DTYPES or w.dtype != dtype:

@@ -76,6 +76,10 @@ def norm_rope(value: torch.Tensor, norm: RMSNorm, pe: tuple[torch.Tensor, torch.
               heads: int) -> torch.Tensor:
     """Weighted RMSNorm over the full width, then split RoPE on the normalized value; one pass
     when the shape allows (``attention.py:353-359`` then ``rope.py:18-61``)."""
+    if value.is_cuda and (native := _lib.host()) is not None:
+        cos, sin = (None, None) if pe is None else pe
+        if (out := native.norm(value, norm.weight, norm.eps, cos, sin, heads, _lib._stream())) is not None:
+            return out
     batch, tokens, dim = value.shape
     head_dim = dim // heads
     out = torch.empty((batch, tokens, dim), dtype=value.dtype, device=value.device)
@@ -104,9 +108,13 @@ def norm_rope_qk(q_raw: torch.Tensor, k_raw: torch.Tensor, q_norm: RMSNorm, k_no
                  pe: tuple[torch.Tensor, torch.Tensor], heads: int):
     """``(norm_rope(q), norm_rope(k))`` for Q and K of the same tokens and tables in one pass
     (the tables are read once); None when the fused kernel does not take the shape."""
+    cos, sin = pe
+    if q_raw.is_cuda and q_norm.eps == k_norm.eps and (native := _lib.host()) is not None:
+        both = native.norm_qk(q_raw, k_raw, q_norm.weight, k_norm.weight, q_norm.eps, cos, sin, heads, _lib._stream())
+        if both is not None:
+            return both
     batch, tokens, dim = q_raw.shape
     head_dim = dim // heads
-    cos, sin = pe
     if (head_dim not in (64, 128) or q_norm.weight is None or k_norm.weight is None or q_norm.eps != k_norm.eps
             or q_norm.weight.dtype != k_norm.weight.dtype or not (cos.dim() == 4 and cos.shape[1] == heads
             and cos.shape[2] == tokens and cos.shape[3] * 2 == head_dim and cos.shape[0] in (1, batch)

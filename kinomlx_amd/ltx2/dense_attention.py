@@ -138,6 +138,11 @@ def batched_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, head
     buffer the next projection reads. With ``kv_heads`` (grouped-query attention) k and v hold
     ``kv_heads * dim`` columns and query head ``h`` reads key/value head
     ``h // (heads // kv_heads)``. ``mask`` is the SDPA mask (``score_bias``)."""
+    if mask is None and q.is_cuda and (native := _lib.host()) is not None:
+        result = native.attention(q, k, v, heads, heads if kv_heads is None else kv_heads, gate, scale, out,
+                                  _lib._stream())
+        if result is not None:
+            return result
     if q.dim() != 3 or k.dim() != 3 or v.shape != k.shape or q.shape[0] != k.shape[0]:
         raise ValueError("batched attention needs (batch, tokens, heads * dim) q, k and v")
     width = q.shape[-1]

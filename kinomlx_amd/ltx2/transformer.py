@@ -67,6 +67,14 @@ def _norm_out_dtype(value: torch.Tensor, out_dtype: torch.dtype | None, what: st
     return dtype
 
 
+def _native_norm(value, shift, scale, eps: float, kind: int, out_dtype):
+    """The modulated norm through the native launch path; None when it leaves the call to Python."""
+    if not value.is_cuda or (native := _lib.host()) is None:
+        return None
+    code = _lib.DTYPE_CODES.get(out_dtype)
+    return None if code is None else native.adaln(value, shift, scale, eps, kind, code, _lib._stream())
+
+
 def adaln(value: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor, eps: float,
           out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """``rms_norm(x) * (1 + scale) + shift`` in one FP32 pass (``transformer.py:16-23``).
@@ -74,6 +82,8 @@ def adaln(value: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor, eps: fl
     or fp16, or an FP32 residual stream; the result is the 16-bit type the next GEMM reads:
     ``value``'s own (as the reference returns ``value.dtype``), or ``out_dtype`` for a stream
     (default bf16)."""
+    if (out := _native_norm(value, shift, scale, eps, _lib.KX_NORM_RMS, out_dtype)) is not None:
+        return out
     out = torch.empty(value.shape, dtype=_norm_out_dtype(value, out_dtype, "adaln"), device=value.device)
     if value.numel():
         shift32, scale32 = _mod_pair(shift, scale)
@@ -86,6 +96,8 @@ def layer_norm_modulate(value: torch.Tensor, shift: torch.Tensor, scale: torch.T
     """``layer_norm(x) * (1 + scale) + shift`` in one FP32 pass (FLUX.2 ``normalized``,
     ``kinomlx/models/flux2/transformer.py:56-57``). ``value`` is bf16 or fp16, or an FP32
     residual stream; the result's type is chosen as ``adaln``'s."""
+    if (out := _native_norm(value, shift, scale, eps, _lib.KX_NORM_LAYER, out_dtype)) is not None:
+        return out
     out = torch.empty(value.shape, dtype=_norm_out_dtype(value, out_dtype, "layer_norm_modulate"),
                       device=value.device)
     if value.numel():
@@ -104,6 +116,9 @@ def gated_residual(value: torch.Tensor, residual: torch.Tensor, gate_value: torc
 
 def modulate(value: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor) -> torch.Tensor:
     """``x * (1 + scale) + shift`` (``transformer.py:33-34``)."""
+    if value.is_cuda and (native := _lib.host()) is not None:
+        if (out := native.modulate(value, shift, scale, _lib._stream())) is not None:
+            return out
     out = torch.empty(value.shape, dtype=value.dtype, device=value.device)
     if value.numel():
         shift32, scale32 = _mod_pair(shift, scale)
