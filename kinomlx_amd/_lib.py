@@ -658,8 +658,9 @@ def tail_split(m: int, n: int, k: int) -> tuple[int, int] | None:
 def splitk_splits(m: int, n: int, k: int) -> int:
     """K slices of a product (1: none): the count the library's cost rule finds fastest with the
     reduction of the partial products included (``kx_gemm_splits``). A few-column product of many
-    rows keeps one slice, so that its rows sum in the same order however many of them a call has."""
-    if n <= 64 or n % 4 or k < 1024 or k % 64 or (m > 512 and n < 1024):
+    rows keeps one slice, so that its rows sum in the same order however many of them a call has; 4 rows
+    and fewer run on a kernel of their own that shares K within a workgroup."""
+    if m <= 4 or n <= 64 or n % 4 or k < 1024 or k % 64 or (m > 512 and n < 1024):
         return 1
     tiles = -(-m // 64) * -(-n // 128)
     if tiles <= 32 and k >= 8192:

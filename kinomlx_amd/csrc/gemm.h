@@ -64,6 +64,12 @@ void launch_dense_slices(bool half, const uint16_t* a, int64_t lda, const uint16
 // The bf16 product with the epilogue's column forms (256-column tiles).
 void launch_dense_columns(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, void* c, int64_t ldc, int m,
                           int n, int k, const Epilogue& epi, hipStream_t s);
+// ---- few rows (gemm_rows.hip) -------------------------------------------------------------------
+
+// c = epilogue(a w^T) for 1 <= m <= FEW_ROWS, k % 8 == 0 and 16-byte aligned rows.
+constexpr int FEW_ROWS = 4;
+void launch_few_rows(bool half, const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, void* c, int64_t ldc,
+                     int m, int n, int k, const Epilogue& epi, hipStream_t s);
 
 namespace {
 

@@ -1217,6 +1217,10 @@ int dispatch(const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, Qua
              hipStream_t s) {
   const char* legacy = getenv("KX355_GEMM_TILE");
   const bool use_legacy = legacy && *legacy;
+  if (QB == 0 && m <= FEW_ROWS && !use_legacy) {
+    launch_few_rows(H, a, lda, w, ldw, c, ldc, (int)m, (int)n, (int)k, epi, s);
+    return KX_OK;
+  }
   if (n <= 64 && k % 128 == 0 && !use_legacy) {
     launch_skinny<QB, H>(a, lda, w, ldw, qw, c, ldc, (int)m, (int)n, (int)k, epi, s);
     return KX_OK;
@@ -1760,7 +1764,7 @@ extern "C" int kx_gemm_splits(int64_t m, int64_t n, int64_t k, int* splits) {
   KX_REQUIRE(splits, "kx_gemm_splits: null result");
   KX_REQUIRE(m >= 0 && n >= 0 && k > 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 30),
              "kx_gemm_splits: bad shape (%lld, %lld, %lld)", (long long)m, (long long)n, (long long)k);
-  *splits = m == 0 || n == 0 || n % 4 || k % DENSE_BK ? 1 : dense_splits(m, n, k);
+  *splits = m <= FEW_ROWS || n == 0 || n % 4 || k % DENSE_BK ? 1 : dense_splits(m, n, k);
   return KX_OK;
 }
 

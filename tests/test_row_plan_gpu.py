@@ -54,10 +54,11 @@ def test_row_split_of_the_norm_rope_projection_reads_its_own_table_rows(device, 
 
 
 def test_split_rule_is_a_pure_function_of_the_sizes():
-    for m, n, k in [(480, 4096, 16384), (1111, 4096, 16384), (1, 4096, 4096)]:
+    for m, n, k in [(480, 4096, 16384), (1111, 4096, 16384), (5, 4096, 4096)]:
         s = _lib.splitk_splits(m, n, k)
         assert s > 1 and k % (64 * s) == 0 and k // s >= 256
     assert _lib.splitk_splits(4608, 512, 8192) == 1  # few columns, many rows: one summation order
     assert _lib.splitk_splits(1111, 16384, 4096) == 1
+    assert _lib.splitk_splits(4, 4096, 16384) == 1  # the few-row kernel
     with pytest.raises(_lib.KernelError):
         _lib.splitk_splits(1 << 31, 4096, 4096)
