@@ -9,7 +9,7 @@
 // K and V tiles of 64 keys go from global memory straight into LDS with buffer_load_dwordx4 ... lds
 // (no VGPR staging) through a ring of 4 stages. Waves 0-7 each issue 1/8 of a stage's DMA
 // instructions; one workgroup barrier per tile makes a tile visible and frees an older buffer.
-// At D = 128 without a score bias the key loop is software-pipelined over 32-key blocks (the next
+// At D = 128 without a bias per query the key loop is software-pipelined over 32-key blocks (the next
 // block's score MFMAs run beside this block's exps, the P V MFMAs beside the next block's max) and
 // tile i+1 becomes visible in the middle of tile i, with tile i+2 in flight; the other forms keep
 // one tile per iteration with tiles i+1 .. i+3 in flight.
@@ -35,6 +35,8 @@
 // Keys past the end are masked to -inf; queries past the end run on a clamped row and are not
 // stored. An optional per-(query, head) gate multiplies the output before the single bf16 rounding.
 #include <math.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -149,6 +151,14 @@ __device__ __forceinline__ void store_o_row(uint16_t* orow, const f32x16 (&o)[DB
 // the row has seen is removed, so that a fully masked row averages V uniformly, as the
 // reference's equal finite scores do. (The sentinel's p is selected, not computed: the FMA of
 // the exp2 argument would leave the rounding error of -1e30 * scale, ~1e21, in the exponent.)
+//
+// A bias that is the same for every query (qs = 0: a padded prompt's mask) takes the pipelined form
+// at D = 128 when its keys fit KEY_BIAS: the workgroup converts it once to fp32 in LDS. A removed
+// key's entry is -2^100 there: the raw score is far below its ulp, and its product with the scale is exact, so
+// that a row of removed keys needs no selection (each p is 2^0).
+constexpr int KEY_BIAS = 4096;  // keys (16 KB of LDS beside the ring)
+constexpr float REMOVED = -0x1p100f;
+enum BiasForm { BIAS_NONE = 0, BIAS_FULL = 1, BIAS_KEYS = 2 };
 struct ScoreBias {
   const uint16_t* ptr;
   int64_t bs, hs, qs;
@@ -164,17 +174,18 @@ struct SplitOut {
   int chunk;  // keys per slice, a multiple of BKV
 };
 
-// RES (D = 128, no bias, no split, at most NSTAGE key tiles): every key tile is copied into LDS
+// RES (D = 128, no full bias, no split, at most NSTAGE key tiles): every key tile is copied into LDS
 // once and stays there while the workgroup runs up to qpw consecutive query tiles of its head; the
 // waves need no barrier after the copy, so one wave's query load and output store overlap the
 // other waves' products.
-template <bool H, int D, bool BIAS, bool SPLIT, bool RES = false>
+template <bool H, int D, int BIAS, bool SPLIT, bool RES = false>
 __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
     const uint16_t* __restrict__ Q, int64_t ldq, const uint16_t* __restrict__ K, int64_t ldk,
     const uint16_t* __restrict__ V, int64_t ldv, uint16_t* __restrict__ O, int64_t ldo, int tq,
     int tk_all, int heads, int kv_group, float scale_log2, const uint16_t* __restrict__ gate,
     int64_t ld_gate, int qtiles, int qpw, ScoreBias bias, SplitOut split) {
-  static_assert(!RES || (D == 128 && !BIAS && !SPLIT), "resident keys: the pipelined form only");
+  static_assert(!RES || (D == 128 && BIAS != BIAS_FULL && !SPLIT), "resident keys: the pipelined form only");
+  static_assert(BIAS != BIAS_KEYS || D == 128, "a bias in LDS: the pipelined form only");
   constexpr int ROWB = D * 2;             // bytes per K / V row
   constexpr int CPR = ROWB / 16;          // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;           // rows per DMA instruction
@@ -185,8 +196,9 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
   static_assert(PER * NDMA == INST, "DMA split");
   const bool dma_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < NDMA;
   constexpr int QS = D / 16, DB = D / 32;
-  constexpr bool PIPE = D == 128 && !BIAS;  // the software-pipelined key loop
+  constexpr bool PIPE = D == 128 && BIAS != BIAS_FULL;  // the software-pipelined key loop
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NSTAGE * STAGE];
+  __shared__ __attribute__((aligned(16))) float key_bias[BIAS != BIAS_KEYS ? 4 : RES ? NSTAGE * BKV : KEY_BIAS];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -286,6 +298,14 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
     // finished its P V products), which takes tile t + NSTAGE - 2. (A ring of 5 with a barrier per
     // two tiles measured 2-3 % slower.)
     auto buf = [&](int t) { return smem + (t % NSTAGE) * STAGE; };
+    if constexpr (BIAS == BIAS_KEYS) {
+      const uint16_t* brow = bias.ptr + (int64_t)b * bias.bs + (int64_t)h * bias.hs + j_begin;
+      for (int i = tid; i < ntiles * BKV; i += NWAVE * 64) {
+        const float add = i < tk ? e2f<H>(brow[i]) * bias.mul : 0.0f;
+        key_bias[i] = add < -1e20f ? REMOVED : add;
+      }
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): written before the first barrier
+    }
     if constexpr (!RES) {
 #pragma unroll
       for (int p = 0; p < NSTAGE - 2; ++p) issue(buf(p), min(p, ntiles - 1) * BKV);
@@ -305,6 +325,15 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
     auto vfrag = [&](const uint8_t* tile, int db, int ts16) {
       return read_vt(tile + (voff0 ^ (db << 6)) + ts16 * 16 * ROWB, 8 * ROWB);
     };
+    // the bias of group g's four keys (elements 4 g .. 4 g + 3) added to block c's scores; keys past the
+    // end have a zero entry
+    auto add_bias = [&](f32x16& sc, int c, int g) {
+      if constexpr (BIAS == BIAS_KEYS) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(key_bias + 32 * c + 8 * g + 4 * lhalf);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[4 * g + e] += v[e];
+      }
+    };
     // keys past the end of block c score -inf
     auto mask = [&](f32x16& sc, int c) {
       if (32 * (c + 1) > tk) {
@@ -317,8 +346,8 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
     f32x16 sc;    // the current block's scores
     float mc;     // the running max in the exp2 domain
     bf16x8 kpre;  // the next step's first K fragment, read ahead where no barrier comes between
-    // the read-ahead of kpre: the streaming forms (the resident form has no registers to spare)
-    constexpr bool PRE = !RES;
+    // the read-ahead of kpre: the streaming forms without a bias (the others have no registers to spare)
+    constexpr bool PRE = !RES && BIAS == BIAS_NONE;
     // block 0's scores and the running max they start
     auto first_block = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -327,6 +356,8 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
       for (int st = 0; st < QS; ++st)
         sc = mfma32x32x16<H>(kfrag(buf(0), 0, st), qf[st], sc);
       mask(sc, 0);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) add_bias(sc, 0, g);
       float tmax = sc[0];
 #pragma unroll
       for (int e = 1; e < 16; ++e) tmax = fmaxf(tmax, sc[e]);
@@ -365,8 +396,9 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
       // exps of elements 0..PA-1 between the 8 score MFMAs, the rest between the 4 P V MFMAs of
       // the first 16 keys (which need only elements 0..7), the max of block cn between the last 4
       // (8, 9, 12 or 14 here leave a query fragment spilled and reloaded in the loop, whose wait
-      // on vmcnt also waits for the K/V copies in flight: 10 % slower; 10 and 11 fit)
-      constexpr int PA = 10;
+      // on vmcnt also waits for the K/V copies in flight: 10 % slower; 10 and 11 fit. With a bias per key 9
+      // is what fits.)
+      constexpr int PA = BIAS == BIAS_KEYS && !RES ? 9 : 10;
       // K fragments are read KFD MFMAs ahead, V fragments VFD ahead (the first ones during the last
       // score MFMAs)
       constexpr int KFD = 1, VFD = 1;
@@ -385,6 +417,13 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
       mask(sn, cn);
+      if constexpr (!RES) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          add_bias(sn, cn, g);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
       // O^T += V^T P^T over the block's two 16-key steps
       float tmax = -INFINITY;
       __builtin_amdgcn_sched_barrier(0);
@@ -399,6 +438,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
         const bf16x8 pb = __builtin_bit_cast(bf16x8, make_uint4(pw[ts][0], pw[ts][1], pw[ts][2], pw[ts][3]));
         o[db] = mfma32x32x16<H>(vf[q % (VFD + 1)], pb, o[db]);
         if (q < DB) {
+          if constexpr (RES) add_bias(sn, cn, q);  // a group per product: four registers for that long only
 #pragma unroll
           for (int e = PA + q * (16 - PA) / DB; e < PA + (q + 1) * (16 - PA) / DB; ++e) pexp(e);
         } else {
@@ -498,7 +538,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
         }
       }
       const int j0 = it * BKV;
-      if constexpr (BIAS) {
+      if constexpr (BIAS == BIAS_FULL) {
         // lane: query qrow, keys j0 + 32 kb + 8 g + 4 lhalf + (0..3) = elements 4 g .. 4 g + 3
         const uint16_t* brow =
             bias.ptr + (int64_t)b * bias.bs + (int64_t)h * bias.hs + (int64_t)qrow * bias.qs + j_begin;
@@ -554,7 +594,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
       bf16x8 pb[2][2];
       auto pexp = [&](int kb, int hf, int e) {
         float p = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * hf + e], scale_log2, -mc));
-        if constexpr (BIAS) p = s[kb][8 * hf + e] == -1e30f ? removed_p : p;
+        if constexpr (BIAS == BIAS_FULL) p = s[kb][8 * hf + e] == -1e30f ? removed_p : p;
         pb[kb][hf][e] = e16<H>(p);
       };
 #pragma unroll
@@ -641,7 +681,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
   *reinterpret_cast<uint2*>(O + ((int64_t)b * tq + q) * ldo + (int64_t)h * D + d) = w2;
 }
 
-template <bool H, int D, bool BIAS, bool SPLIT, bool RES = false>
+template <bool H, int D, int BIAS, bool SPLIT, bool RES = false>
 void launch_attn_t(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o,
                    int64_t ldo, int64_t tq, int64_t tk, int64_t heads, int64_t kv_heads, float scale,
                    const void* gate, int64_t ld_gate, ScoreBias bias, SplitOut split, dim3 grid, int qtiles,
@@ -677,28 +717,43 @@ int launch_attn(const void* q, int64_t ldq, const void* k, int64_t ldk, const vo
   const int qtiles = (int)((tq + BQ - 1) / BQ);
   const int64_t blocks = (int64_t)qtiles * heads * batch;
   const dim3 grid((unsigned)blocks, (unsigned)splits);
+  // One bias row for all queries goes through LDS and keeps the pipelined form (a padded prompt's mask, 32
+  // heads: 9216 queries x 256 keys 133 -> 57 us, 16384 x 1024 684 -> 318, 1000 x 100 24 -> 16). The scale's
+  // range keeps the removed keys' -2^100 times the scale finite and below every score.
+  const int64_t slice = splits > 1 ? split.chunk : tk;
+  const bool keys = D == 128 && bias.ptr && (bias.qs == 0 || tq == 1) && slice <= KEY_BIAS && scale >= 0x1p-20f &&
+                    scale <= 0x1p20f;
+  const auto launch = [&](auto form, auto is_split, auto resident, dim3 g, int qpw) {
+    launch_attn_t<H, D, decltype(form)::value, decltype(is_split)::value, decltype(resident)::value>(
+        q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale, gate, ld_gate, bias, split, g, qtiles, s, qpw);
+  };
+  // the keys form exists at D = 128 only (`keys` is false otherwise)
+  constexpr std::integral_constant<int, BIAS_NONE> none{};
+  constexpr std::integral_constant<int, BIAS_FULL> full{};
+  constexpr std::integral_constant<int, D == 128 ? BIAS_KEYS : BIAS_FULL> by_key{};
+  constexpr std::false_type no{};
+  constexpr std::true_type yes{};
   if (splits > 1) {
-    if (bias.ptr)
-      launch_attn_t<H, D, true, true>(q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale, gate, ld_gate,
-                                   bias, split, grid, qtiles, s);
-    else
-      launch_attn_t<H, D, false, true>(q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale, gate, ld_gate,
-                                    bias, split, grid, qtiles, s);
+    if (keys) launch(by_key, yes, no, grid, 1);
+    else if (bias.ptr) launch(full, yes, no, grid, 1);
+    else launch(none, yes, no, grid, 1);
     const int64_t rows = batch * heads * tq;
     attn_combine_kernel<H, D><<<(unsigned)((rows * (D / 4) + 255) / 256), 256, 0, s>>>(
         split.o, split.ml, splits, rows, (int)tq, (int)heads, (uint16_t*)o, ldo, (const uint16_t*)gate, ld_gate);
-  } else if (bias.ptr) {
-    launch_attn_t<H, D, true, false>(q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale, gate, ld_gate,
-                                  bias, split, grid, qtiles, s);
+  } else if (bias.ptr && !keys) {
+    launch(full, no, no, grid, 1);
   } else if (D == 128 && tk <= NSTAGE * BKV) {
     // few keys (a text context): they stay in LDS while a workgroup runs several query tiles
     const int qpw = resident_qpw(qtiles, heads * batch);
     const dim3 rgrid((unsigned)((qtiles + qpw - 1) / qpw * heads * batch));
-    launch_attn_t<H, D, false, false, D == 128>(q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale, gate,
-                                             ld_gate, bias, split, rgrid, qtiles, s, qpw);
+    constexpr std::integral_constant<bool, D == 128> resident{};
+    constexpr std::integral_constant<int, D == 128 ? BIAS_KEYS : BIAS_NONE> by_key_res{};
+    if (keys) launch(by_key_res, no, resident, rgrid, qpw);
+    else launch(none, no, resident, rgrid, qpw);
+  } else if (keys) {
+    launch(by_key, no, no, grid, 1);
   } else {
-    launch_attn_t<H, D, false, false>(q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale, gate, ld_gate,
-                                   bias, split, grid, qtiles, s);
+    launch(none, no, no, grid, 1);
   }
   return check_launch(ename<H>("kx_attention_fwd_bf16", "kx_attention_fwd_f16"));
 }
