@@ -348,7 +348,7 @@ def main() -> int:
 
 
 _DISPATCHES = {"kx_gemm_splitk_bf16": 2, "kx_gemm_splitk_noalloc_bf16": 2, "kx_attention_split_fwd_bf16": 2,
-               "kx_all_finite": 2}
+               "kx_attention_tail_fwd_bf16": 2, "kx_all_finite": 2}
 
 
 def profile_summary(root: str, warmup: int = 0) -> int:

@@ -123,6 +123,18 @@ int kx_attention_split_fwd_bf16(const void* q, int64_t ldq, const void* k, int64
                                 int splits, kx_stream_t stream);
 
 /*
+ * kx_attention_gqa_fwd_bf16 for 128-wide heads whose query tiles (384 queries of one head) fill whole
+ * rounds of 256 workgroups and a part of one more: the whole rounds run as always, the tiles past
+ * them as `splits` (2..16) key slices in the same launch, merged by one pass over the workspace (splits *
+ * (tiles past the whole rounds) * 384 * (head_dim + 2) floats, caller-owned). Same result up to the
+ * order of those tiles' fp32 sums. Refuses calls without a whole round or without a rest.
+ */
+int kx_attention_tail_fwd_bf16(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                               void* o, int64_t ldo, int64_t batch, int64_t tq, int64_t tk, int64_t heads,
+                               int64_t kv_heads, int64_t head_dim, float scale, const void* gate, int64_t ld_gate,
+                               void* workspace, int64_t workspace_bytes, int splits, kx_stream_t stream);
+
+/*
  * Split-half RoPE, standalone: replaces split_rope.rotate (kinomlx/kernels/split_rope.py:144-163,
  * arithmetic :35-56). x/y are (batch, tokens, heads * 2 * half) rows at stride ldx/ldy; tables
  * token-major (table_batch, tokens, heads * half), table_batched selects per-batch tables.
@@ -563,6 +575,10 @@ int kx_attention_split_fwd_f16(const void* q, int64_t ldq, const void* k, int64_
                                int64_t ld_gate, const void* bias, int64_t bias_bs, int64_t bias_hs,
                                int64_t bias_qs, void* workspace, int64_t workspace_bytes, int splits,
                                kx_stream_t stream);
+int kx_attention_tail_fwd_f16(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                              void* o, int64_t ldo, int64_t batch, int64_t tq, int64_t tk, int64_t heads,
+                              int64_t kv_heads, int64_t head_dim, float scale, const void* gate, int64_t ld_gate,
+                              void* workspace, int64_t workspace_bytes, int splits, kx_stream_t stream);
 int kx_gemm_f16(const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias, void* c, int64_t ldc,
                 int64_t m, int64_t n, int64_t k, int epilogue, const void* resid, int64_t ldr, const float* gate,
                 int64_t gate_div, int64_t gate_stride, kx_stream_t stream);

@@ -83,6 +83,9 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _I64, _P, _I64, _I64,
         _I64, _P, _I64, _I, _P,
     ],
+    "kx_attention_tail_fwd_bf16": [
+        _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _I64, _P, _I64, _I, _P,
+    ],
     "kx_gemm_bf16": [
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _I64, _P,
     ],
@@ -137,7 +140,8 @@ SIGNATURES: dict[str, list] = {
 # fp16 entry points: the bf16 namesake's arguments with fp16 16-bit tensors (include/kx355.h)
 F16_ENTRIES = (
     "kx_adaln_norm", "kx_rmsnorm_rope", "kx_qk_rmsnorm_rope", "kx_qk_rmsnorm_rope_h64", "kx_rope_split", "kx_rope_pair",
-    "kx_attention_fwd", "kx_attention_gqa_fwd", "kx_attention_bias_fwd", "kx_attention_split_fwd", "kx_gemm",
+    "kx_attention_fwd", "kx_attention_gqa_fwd", "kx_attention_bias_fwd", "kx_attention_split_fwd",
+    "kx_attention_tail_fwd", "kx_gemm",
     "kx_gemm_splitk", "kx_gelu_tanh", "kx_silu", "kx_swiglu", "kx_modulate", "kx_gated_residual",
 )
 for _base in F16_ENTRIES:
@@ -193,7 +197,7 @@ def _bind_host():
         raise RuntimeError(f"the native launch path is not built ({exc}); run `python -m kinomlx_amd.csrc.build`") from exc
     names = [*SIGNATURES, "kx_last_error"]
     module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names}, KernelError,
-                gemm_plan, lambda batch, tq, tk, heads: (0, attention_splits(batch, tq, tk, heads)))
+                gemm_plan, lambda *call: (attention_tail(*call), attention_splits(*call)))
     _host = module
     return module
 
@@ -442,6 +446,17 @@ def launch_attention(q, k, v, out, *, batch, tq, tk, heads, head_dim, scale, gat
             _ptr(bias), *(bias_strides or (0, 0, 0)), _ptr(work), work.numel() * 4, splits, _stream(),
         )
         return
+    tail = attention_tail(batch, tq, tk, heads) if head_dim == 128 and bias is None else 1
+    if tail > 1:
+        used = -(-tk // (-(-(-(-tk // tail)) // 64) * 64))
+        rest = -(-tq // 384) * heads * batch % 256
+        work = torch.empty(used * rest * 384 * (head_dim + 2), dtype=torch.float32, device=q.device)
+        _call(
+            f"kx_attention_tail_fwd_{sfx}", _ptr(q), q.stride(-2), _ptr(k), k.stride(-2), _ptr(v), v.stride(-2),
+            _ptr(out), out.stride(-2), batch, tq, tk, heads, kv_heads or heads, head_dim, scale, _ptr(gate), ld_gate,
+            _ptr(work), work.numel() * 4, tail, _stream(),
+        )
+        return
     if bias is not None:
         _call(
             f"kx_attention_bias_fwd_{sfx}", _ptr(q), q.stride(-2), _ptr(k), k.stride(-2), _ptr(v), v.stride(-2),
@@ -471,6 +486,27 @@ def attention_splits(batch: int, tq: int, tk: int, heads: int) -> int:
     if blocks >= 128 or tk < 1024:
         return 1
     return max(1, min(16, -(-512 // blocks), tk // 256))
+
+
+def attention_tail(batch: int, tq: int, tk: int, heads: int) -> int:
+    """Key slices (2 to 4; 1: none) for the query tiles (384 queries x 1 head, 128 wide) past the last whole
+    round of 256 workgroups. A partial round takes as long as one workgroup's whole key loop; cut
+    into ``s`` slices the rest takes ``ceil(rest * s / 256) / s`` of it and a merge of the partial rows. The
+    round's time (0.04 us per key) and the merge's rate (4.5 TB/s over one write and one read, 6 us for the launch)
+    are fitted; measured in us, unsplit / chosen, 32 heads, as many keys as queries: 3500 256 / 209 (4 slices),
+    4608 336 / 312 (2), 6300 702 / 584 (4), 10000 1507 / 1417 (2); a rest of 192 tiles is slower in slices
+    (5376: 415, 452 with 4)."""
+    blocks = -(-tq // 384) * heads * batch
+    rest = blocks % 256
+    if blocks < 256 or rest == 0 or tk < 1024:
+        return 1
+    best, splits = 0.0, 1
+    for s in (2, 3, 4):
+        saved = 0.04 * tk * (1.0 - -(-rest * s // 256) / s)
+        merge = 6.0 + rest * 384 * 128 * 4 * 2 * s / 4.5e6
+        if saved - merge > best:
+            best, splits = saved - merge, s
+    return splits
 
 
 def _dtype_flags(out, resid, name: str, half: torch.dtype = torch.bfloat16) -> int:

@@ -168,17 +168,25 @@ struct ScoreBias {
 // Split over keys (few query tiles, many keys): grid row y takes keys [y * chunk, (y + 1) * chunk)
 // and writes its unnormalized fp32 O rows and (running max in the exp2 domain, row sum) to the
 // workspace; attn_combine_kernel merges the slices.
+//
+// The tail form does so for the last, partial round of workgroups only: the first `full` workgroups
+// (whole rounds of 256) each take all keys and store their rows, the `tail` query tiles that remain run as
+// `tail` workgroups per slice, with BQ partial rows per tile, in the same launch: they start as the last whole
+// round's workgroups end. (4608 tokens x 32 heads, one and a half rounds: 336 -> 312 us; 6300 tokens, two
+// and an eighth: 702 -> 584.)
 struct SplitOut {
-  float* o;   // (splits, batch * heads, tq, D)
-  float* ml;  // (splits, batch * heads, tq, 2)
+  float* o;   // (splits, batch * heads, tq, D); the tail form: (splits, tail, BQ, D)
+  float* ml;  // (splits, batch * heads, tq, 2); the tail form: (splits, tail, BQ, 2)
   int chunk;  // keys per slice, a multiple of BKV
+  int full, tail;
 };
+enum KeySplit { KEYS_ALL = 0, KEYS_SLICES = 1, KEYS_TAIL = 2 };
 
 // RES (D = 128, no full bias, no split, at most NSTAGE key tiles): every key tile is copied into LDS
 // once and stays there while the workgroup runs up to qpw consecutive query tiles of its head; the
 // waves need no barrier after the copy, so one wave's query load and output store overlap the
 // other waves' products.
-template <bool H, int D, int BIAS, bool SPLIT, bool RES = false>
+template <bool H, int D, int BIAS, int SPLIT, bool RES = false>
 __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
     const uint16_t* __restrict__ Q, int64_t ldq, const uint16_t* __restrict__ K, int64_t ldk,
     const uint16_t* __restrict__ V, int64_t ldv, uint16_t* __restrict__ O, int64_t ldo, int tq,
@@ -204,7 +212,23 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lhalf = lane >> 5;
   // work order: XCD-contiguous so the workgroups of one XCD share few heads' K/V in its L2
-  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  int t, part_row = 0;  // the tail form's first partial row of this workgroup
+  bool whole = SPLIT != KEYS_SLICES;
+  int slice = 0;
+  if constexpr (SPLIT == KEYS_TAIL) {
+    whole = (int)blockIdx.x < split.full;
+    if (whole) {
+      t = xcd_remap(blockIdx.x, split.full);
+    } else {
+      const int u = xcd_remap(blockIdx.x - split.full, gridDim.x - split.full);
+      slice = u / split.tail;
+      t = split.full + u % split.tail;
+      part_row = u * BQ;
+    }
+  } else {
+    t = xcd_remap(blockIdx.x, gridDim.x);
+    if constexpr (SPLIT == KEYS_SLICES) slice = blockIdx.y;
+  }
   const int wph = RES ? (qtiles + qpw - 1) / qpw : qtiles;  // workgroups per (batch, head)
   const int qt = RES ? (t % wph) * qpw : t % qtiles, bh = t / wph;
   const int h = bh % heads, b = bh / heads;
@@ -212,8 +236,8 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
   const int hk = h / kv_group;  // grouped-query attention: kv_group query heads share a K/V head
   // this workgroup's keys: all of them, or one slice of the split form
   int j_begin = 0, tk = tk_all;
-  if constexpr (SPLIT) {
-    j_begin = blockIdx.y * split.chunk;
+  if (!whole) {
+    j_begin = slice * split.chunk;
     tk = min(tk_all - j_begin, split.chunk);
   }
   const char* Kb = reinterpret_cast<const char*>(K + ((int64_t)b * tk_all + j_begin) * ldk + (int64_t)hk * D);
@@ -624,38 +648,57 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
   wait_vmcnt<0>();  // the re-read tiles past the end have landed before the workgroup ends
 
   // normalise, gate, store: lane holds query q0 + lrow, dims db*32 + 8g + 4*lhalf + (0..3)
+  // (the tail form reads the lane id again: held across its key loop it would spill a query fragment)
+  int row_in = lrow, half_in = lhalf;
+  if constexpr (SPLIT == KEYS_TAIL) {
+    uint32_t ln;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+    row_in = ln & 31;
+    half_in = ln >> 5;
+  }
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-  const int q = q0 + lrow;
+  const int q = q0 + row_in;
   if (q >= tq) return;
-  if constexpr (SPLIT) {
-    const int64_t row = ((int64_t)blockIdx.y * (gridDim.x / qtiles) + bh) * tq + q;
+  if (!whole) {
+    const int64_t row = SPLIT == KEYS_TAIL ? (int64_t)part_row + wave * 32 + row_in
+                                           : ((int64_t)slice * (gridDim.x / qtiles) + bh) * tq + q;
     float* orow = split.o + row * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<float4*>(orow + db * 32 + 8 * g + 4 * lhalf) =
+        *reinterpret_cast<float4*>(orow + db * 32 + 8 * g + 4 * half_in) =
             make_float4(o[db][4 * g + 0], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]);
-    if (lhalf == 0) *reinterpret_cast<float2*>(split.ml + 2 * row) = make_float2(m_run * scale_log2, l_tot);
+    if (half_in == 0) *reinterpret_cast<float2*>(split.ml + 2 * row) = make_float2(m_run * scale_log2, l_tot);
     return;
   }
   float scale_out = 1.0f / l_tot;
   if (gate) scale_out *= e2f<H>(gate[((int64_t)b * tq + q) * ld_gate + h]);
-  store_o_row<H, DB>(O + ((int64_t)b * tq + q) * ldo + (int64_t)h * D, o, scale_out, lhalf);
+  store_o_row<H, DB>(O + ((int64_t)b * tq + q) * ldo + (int64_t)h * D, o, scale_out, half_in);
 }
 
 // out = (sum_y 2^(m_y - M) O_y) / (sum_y 2^(m_y - M) l_y) * gate, M = max_y m_y: the slices of the
 // split form merged (4 dims of one row per thread).
-template <bool H, int D>
+// The tail form's partial rows are (tile, row of the tile), the tiles from `full` on.
+template <bool H, int D, bool TAIL>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restrict__ part_o,
                                                            const float* __restrict__ part_ml, int splits,
                                                            int64_t rows, int tq, int heads,
                                                            uint16_t* __restrict__ O, int64_t ldo,
-                                                           const uint16_t* __restrict__ gate, int64_t ld_gate) {
+                                                           const uint16_t* __restrict__ gate, int64_t ld_gate,
+                                                           int full, int qtiles) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= rows * (D / 4)) return;
   const int64_t row = idx / (D / 4);  // (b * heads + h) * tq + q
   const int d = (int)(idx - row * (D / 4)) * 4;
+  int q = TAIL ? 0 : (int)(row % tq);
+  int64_t bh = TAIL ? 0 : row / tq;
+  if constexpr (TAIL) {
+    const int64_t tile = full + row / BQ;
+    bh = tile / qtiles;
+    q = (int)(tile % qtiles) * BQ + (int)(row % BQ);
+    if (q >= tq) return;
+  }
   float mx = -INFINITY;
   for (int y = 0; y < splits; ++y) mx = fmaxf(mx, part_ml[2 * (y * rows + row)]);
   float l = 0.0f;
@@ -670,8 +713,6 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     acc.z += w * p.z;
     acc.w += w * p.w;
   }
-  const int q = (int)(row % tq);
-  const int64_t bh = row / tq;
   const int h = (int)(bh % heads), b = (int)(bh / heads);
   float scale_out = 1.0f / l;
   if (gate) scale_out *= e2f<H>(gate[((int64_t)b * tq + q) * ld_gate + h]);
@@ -681,7 +722,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
   *reinterpret_cast<uint2*>(O + ((int64_t)b * tq + q) * ldo + (int64_t)h * D + d) = w2;
 }
 
-template <bool H, int D, int BIAS, bool SPLIT, bool RES = false>
+template <bool H, int D, int BIAS, int SPLIT, bool RES = false>
 void launch_attn_t(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o,
                    int64_t ldo, int64_t tq, int64_t tk, int64_t heads, int64_t kv_heads, float scale,
                    const void* gate, int64_t ld_gate, ScoreBias bias, SplitOut split, dim3 grid, int qtiles,
@@ -731,17 +772,27 @@ int launch_attn(const void* q, int64_t ldq, const void* k, int64_t ldk, const vo
   constexpr std::integral_constant<int, BIAS_NONE> none{};
   constexpr std::integral_constant<int, BIAS_FULL> full{};
   constexpr std::integral_constant<int, D == 128 ? BIAS_KEYS : BIAS_FULL> by_key{};
-  constexpr std::false_type no{};
-  constexpr std::true_type yes{};
-  if (splits > 1) {
-    if (keys) launch(by_key, yes, no, grid, 1);
-    else if (bias.ptr) launch(full, yes, no, grid, 1);
-    else launch(none, yes, no, grid, 1);
+  constexpr std::integral_constant<int, KEYS_ALL> no{};
+  constexpr std::integral_constant<int, KEYS_SLICES> yes{};
+  constexpr std::false_type stream{};
+  if (split.tail) {
+    if constexpr (D == 128) {
+      constexpr std::integral_constant<int, KEYS_TAIL> tail{};
+      launch(none, tail, stream, dim3((unsigned)(split.full + split.tail * splits)), 1);
+      const int64_t rows = (int64_t)split.tail * BQ;
+      attn_combine_kernel<H, D, true><<<(unsigned)((rows * (D / 4) + 255) / 256), 256, 0, s>>>(
+          split.o, split.ml, splits, rows, (int)tq, (int)heads, (uint16_t*)o, ldo, (const uint16_t*)gate, ld_gate,
+          split.full, qtiles);
+    }
+  } else if (splits > 1) {
+    if (keys) launch(by_key, yes, stream, grid, 1);
+    else if (bias.ptr) launch(full, yes, stream, grid, 1);
+    else launch(none, yes, stream, grid, 1);
     const int64_t rows = batch * heads * tq;
-    attn_combine_kernel<H, D><<<(unsigned)((rows * (D / 4) + 255) / 256), 256, 0, s>>>(
-        split.o, split.ml, splits, rows, (int)tq, (int)heads, (uint16_t*)o, ldo, (const uint16_t*)gate, ld_gate);
+    attn_combine_kernel<H, D, false><<<(unsigned)((rows * (D / 4) + 255) / 256), 256, 0, s>>>(
+        split.o, split.ml, splits, rows, (int)tq, (int)heads, (uint16_t*)o, ldo, (const uint16_t*)gate, ld_gate, 0, 1);
   } else if (bias.ptr && !keys) {
-    launch(full, no, no, grid, 1);
+    launch(full, no, stream, grid, 1);
   } else if (D == 128 && tk <= NSTAGE * BKV) {
     // few keys (a text context): they stay in LDS while a workgroup runs several query tiles
     const int qpw = resident_qpw(qtiles, heads * batch);
@@ -751,9 +802,9 @@ int launch_attn(const void* q, int64_t ldq, const void* k, int64_t ldk, const vo
     if (keys) launch(by_key_res, no, resident, rgrid, qpw);
     else launch(none, no, resident, rgrid, qpw);
   } else if (keys) {
-    launch(by_key, no, no, grid, 1);
+    launch(by_key, no, stream, grid, 1);
   } else {
-    launch(none, no, no, grid, 1);
+    launch(none, no, stream, grid, 1);
   }
   return check_launch(ename<H>("kx_attention_fwd_bf16", "kx_attention_fwd_f16"));
 }
@@ -770,7 +821,7 @@ int attention_entry(const char* name, const void* q, int64_t ldq, const void* k,
                     int64_t tk, int64_t heads, int64_t kv_heads, int64_t head_dim, float scale,
                     const void* gate, int64_t ld_gate, kx_stream_t stream,
                     ScoreBias bias = ScoreBias{nullptr, 0, 0, 0, 0.0f},
-                    SplitOut split = SplitOut{nullptr, nullptr, 0}, int splits = 1) {
+                    SplitOut split = SplitOut{nullptr, nullptr, 0, 0, 0}, int splits = 1) {
   KX_REQUIRE(q && k && v && o, "%s: null tensor", name);
   KX_REQUIRE(head_dim == 64 || head_dim == 128, "%s: head_dim must be 64 or 128, got %lld", name,
              (long long)head_dim);
@@ -796,6 +847,35 @@ int attention_entry(const char* name, const void* q, int64_t ldq, const void* k,
                             gate, ld_gate, bias, split, splits, (hipStream_t)stream);
   return launch_attn<H, 64>(q, ldq, k, ldk, v, ldv, o, ldo, batch, tq, tk, heads, kv_heads, scale,
                          gate, ld_gate, bias, split, splits, (hipStream_t)stream);
+}
+
+// The tail form's entry (see SplitOut).
+template <bool H>
+int attention_tail_entry(const char* name, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v,
+                         int64_t ldv, void* o, int64_t ldo, int64_t batch, int64_t tq, int64_t tk, int64_t heads,
+                         int64_t kv_heads, int64_t head_dim, float scale, const void* gate, int64_t ld_gate,
+                         void* workspace, int64_t workspace_bytes, int splits, kx_stream_t stream) {
+  KX_REQUIRE(workspace && aligned16(workspace), "%s: workspace must be a 16-byte aligned buffer", name);
+  KX_REQUIRE(splits >= 2 && splits <= 16, "%s: splits must be 2..16, got %d", name, splits);
+  KX_REQUIRE(head_dim == 128, "%s: head_dim must be 128, got %lld", name, (long long)head_dim);
+  KX_REQUIRE(batch > 0 && tq > 0 && tk > 0 && heads > 0 && batch < (1ll << 31) && tq < (1ll << 30) &&
+                 tk < (1ll << 30) && heads < (1ll << 31),
+             "%s: bad shape", name);
+  const int64_t blocks = (tq + BQ - 1) / BQ * heads * batch;
+  const int64_t full = blocks / 256 * 256, tail = blocks - full;
+  KX_REQUIRE(full > 0 && tail > 0 && blocks < (1ll << 30), "%s: %lld query tiles are not whole rounds and a rest",
+             name, (long long)blocks);
+  const int64_t chunk = ((tk + splits - 1) / splits + BKV - 1) / BKV * BKV;
+  const int used = (int)((tk + chunk - 1) / chunk);
+  const int64_t rows = tail * BQ;
+  KX_REQUIRE(used >= 2, "%s: %lld keys are too few for slices", name, (long long)tk);
+  KX_REQUIRE(workspace_bytes >= used * rows * (head_dim + 2) * 4,
+             "%s: workspace of %lld bytes is below splits * tiles * %d * (head_dim + 2) * 4", name,
+             (long long)workspace_bytes, BQ);
+  float* ws = static_cast<float*>(workspace);
+  const SplitOut split{ws, ws + used * rows * head_dim, (int)chunk, (int)full, (int)tail};
+  return attention_entry<H>(name, q, ldq, k, ldk, v, ldv, o, ldo, batch, tq, tk, heads, kv_heads, head_dim, scale,
+                            gate, ld_gate, stream, ScoreBias{nullptr, 0, 0, 0, 0.0f}, split, used);
 }
 }  // namespace
 
@@ -863,10 +943,23 @@ extern "C" int kx_attention_split_fwd_##SUFFIX(const void* q, int64_t ldq, const
     sb = ScoreBias{(const uint16_t*)bias, bias_bs, bias_hs, bias_qs, 1.0f / scale};                                    \
   }                                                                                                                    \
   float* ws = static_cast<float*>(workspace);                                                                          \
-  const SplitOut split{ws, ws + (int64_t)used * rows * head_dim, (int)chunk};                                          \
+  const SplitOut split{ws, ws + (int64_t)used * rows * head_dim, (int)chunk, 0, 0};                                          \
   return attention_entry<H>(name, q, ldq, k, ldk, v, ldv, o, ldo, batch, tq, tk, heads, kv_heads, head_dim, scale,     \
                          gate, ld_gate, stream, sb, split, used);                                                      \
 }                                                                                                                      \
 
 KX_ATTN_ENTRY(bf16, false)
 KX_ATTN_ENTRY(f16, true)
+
+#define KX_ATTN_TAIL_ENTRY(SUFFIX, H)                                                                                 \
+  extern "C" int kx_attention_tail_fwd_##SUFFIX(                                                                      \
+      const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o, int64_t ldo,       \
+      int64_t batch, int64_t tq, int64_t tk, int64_t heads, int64_t kv_heads, int64_t head_dim, float scale,          \
+      const void* gate, int64_t ld_gate, void* workspace, int64_t workspace_bytes, int splits, kx_stream_t stream) {  \
+    return attention_tail_entry<H>("kx_attention_tail_fwd_" #SUFFIX, q, ldq, k, ldk, v, ldv, o, ldo, batch, tq, tk,   \
+                                   heads, kv_heads, head_dim, scale, gate, ld_gate, workspace, workspace_bytes,       \
+                                   splits, stream);                                                                   \
+  }
+
+KX_ATTN_TAIL_ENTRY(bf16, false)
+KX_ATTN_TAIL_ENTRY(f16, true)

@@ -33,6 +33,7 @@ struct Api {
   decltype(&kx_qk_rmsnorm_rope_bf16) qk128[2], qk64[2];
   decltype(&kx_attention_gqa_fwd_bf16) attention[2];
   decltype(&kx_attention_split_fwd_bf16) attention_split[2];
+  decltype(&kx_attention_tail_fwd_bf16) attention_tail[2];
   decltype(&kx_gemm_columns_bf16) columns;
   decltype(&kx_table_add_f32) table_add;
   decltype(&kx_last_error) last_error;
@@ -40,7 +41,7 @@ struct Api {
 
 PyObject* kernel_error = nullptr;    // the exception of a failed entry point
 PyObject* gemm_plan_fn = nullptr;    // (m, n, k) -> (head rows or 0, splits)
-PyObject* attn_plan_fn = nullptr;    // (batch, tq, tk, heads) -> splits
+PyObject* attn_plan_fn = nullptr;    // (batch, tq, tk, heads) -> (slices of the tail, slices)
 
 struct Refused {};  // raised inside a function: return None to the Python caller
 struct PyFailed {};  // a Python error is set
@@ -410,13 +411,20 @@ Tensor attention(PyObject* const* a) {
   }
   const int h = type == at::kHalf;
   const float scale = a[6] == Py_None ? (float)std::pow((double)dim, -0.5) : real(a[6]);
-  const int64_t splits = plan(attn_plans, attn_plan_fn, {batch, tq, tk, heads}, 4)[1];
+  const auto [tail, splits] = plan(attn_plans, attn_plan_fn, {batch, tq, tk, heads}, 4);
   if (splits > 1) {
     const int64_t chunk = ((tk + splits - 1) / splits + 63) / 64 * 64, used = (tk + chunk - 1) / chunk;
     const Tensor work = floats(q, used * batch * heads * tq * (dim + 2));
     call("kx_attention_split_fwd", api.attention_split[h], ptr(q), q.stride(1), ptr(k), k.stride(1), ptr(v),
          v.stride(1), ptr(out), out.stride(1), batch, tq, tk, heads, kv, dim, scale, ptr(gate), ld_gate, nullptr,
          0, 0, 0, ptr(work), work.numel() * 4, (int)splits, stream);
+  } else if (tail > 1 && dim == 128) {
+    const int64_t chunk = ((tk + tail - 1) / tail + 63) / 64 * 64, used = (tk + chunk - 1) / chunk;
+    const int64_t rest = (tq + 383) / 384 * heads * batch % 256;
+    const Tensor work = floats(q, used * rest * 384 * (dim + 2));
+    call("kx_attention_tail_fwd", api.attention_tail[h], ptr(q), q.stride(1), ptr(k), k.stride(1), ptr(v), v.stride(1),
+         ptr(out), out.stride(1), batch, tq, tk, heads, kv, dim, scale, ptr(gate), ld_gate, ptr(work),
+         work.numel() * 4, (int)tail, stream);
   } else {
     call("kx_attention_gqa_fwd", api.attention[h], ptr(q), q.stride(1), ptr(k), k.stride(1), ptr(v), v.stride(1),
          ptr(out), out.stride(1), batch, tq, tk, heads, kv, dim, scale, ptr(gate), ld_gate, stream);
@@ -500,6 +508,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t count) {
     both(a.qk64[h], "kx_qk_rmsnorm_rope_h64_");
     both(a.attention[h], "kx_attention_gqa_fwd_");
     both(a.attention_split[h], "kx_attention_split_fwd_");
+    both(a.attention_tail[h], "kx_attention_tail_fwd_");
   }
   get(a.columns, "kx_gemm_columns_bf16");
   get(a.table_add, "kx_table_add_f32");
