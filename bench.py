@@ -266,7 +266,7 @@ def main() -> int:
         per_block = len(records) // args.steps
         with open(args.launch_log, "w") as fh:
             json.dump([{"label": _kernel_label(n, a), "entry": n, "flops": _kernel_flops(n, a),
-                        "bytes": _kernel_bytes(n, a)} for n, a, _ in records[:per_block]], fh, indent=1)
+                        "bytes": _kernel_bytes(n, a), "kernels": _kernel_count(n, a)} for n, a, _ in records[:per_block]], fh, indent=1)
     dominant = max(kernel_ms_per_step, key=kernel_ms_per_step.get)
     dom_avg_ms = statistics.mean(per_kernel[dominant])
     dom_tflops = flops_of[dominant] / (dom_avg_ms * 1e-3) / 1e12
@@ -347,6 +347,21 @@ def main() -> int:
     return 0
 
 
+def _kernel_count(name: str, args: tuple) -> int:
+    """Kernels that one launch runs: the split forms add their reduction / merge pass, the finite check its
+    flag initialisation, and a dense product can split its rows over two tile sizes."""
+    if name == "kx_gemm_bf16":
+        import ctypes
+
+        from kinomlx_amd import _lib
+
+        count = ctypes.c_int(1)
+        if _lib.load().kx_gemm_kernels(args[7], args[8], args[9], ctypes.addressof(count)):
+            raise RuntimeError(f"kx_gemm_kernels refused {args[7:10]}")
+        return count.value
+    return _DISPATCHES.get(name, 1)
+
+
 _DISPATCHES = {"kx_gemm_splitk_bf16": 2, "kx_gemm_splitk_noalloc_bf16": 2, "kx_attention_split_fwd_bf16": 2,
                "kx_attention_tail_fwd_bf16": 2, "kx_all_finite": 2}
 
@@ -365,11 +380,10 @@ def profile_summary(root: str, warmup: int = 0) -> int:
 
     with open(os.path.join(root, "launches.json")) as fh:
         launches = json.load(fh)
-    # kernel dispatches per launch: the split forms add their reduction / merge pass, the finite
-    # check its flag initialisation
+    # kernel dispatches per launch (logs without the count: the entry point's usual one)
     groups, period = [], 0
     for entry in launches:
-        count = _DISPATCHES.get(entry.get("entry", ""), 1)
+        count = entry.get("kernels", _DISPATCHES.get(entry.get("entry", ""), 1))
         groups.append(range(period, period + count))
         period += count
 

@@ -247,6 +247,10 @@ int kx_gemm_splitk_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, 
  * kx_gemm_bf16, more for kx_gemm_splitk_bf16 with a workspace of splits * m * n * 4 bytes. A pure
  * function of the sizes; no GPU call. */
 int kx_gemm_splits(int64_t m, int64_t n, int64_t k, int* splits);
+
+/* *count = the kernels that one kx_gemm_bf16 call of these sizes launches (2 where its rows are split over two
+ * tile sizes), for readers of a kernel trace. A pure function of the sizes; no GPU call. */
+int kx_gemm_kernels(int64_t m, int64_t n, int64_t k, int* count);
 /* Size of the static device array kx_gemm_splitk_noalloc_bf16 keeps its partial products in. */
 #define KX_SPLITK_SCRATCH_BYTES (16ll << 20)
 

@@ -93,6 +93,7 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _I64, _P, _I64, _I, _P,
     ],
     "kx_gemm_splits": [_I64, _I64, _I64, _P],
+    "kx_gemm_kernels": [_I64, _I64, _I64, _P],
     "kx_gemm_splitk_noalloc_bf16": [
         _P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _I64, _I, _P,
     ],

@@ -56,6 +56,8 @@ bool rows_last_first(int64_t m, int64_t k);
 // (KX355_GEMM_LDS_TILE = 0 .. 3 forces one tile size).
 void launch_dense(bool half, const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, void* c, int64_t ldc,
                   int m, int n, int k, const Epilogue& epi, hipStream_t s);
+// The kernels that launch_dense runs for these sizes (2 with a row split).
+int dense_kernels(int64_t m, int64_t n, int64_t k);
 // The K slices (1, 2, 4, 8 or 16) in which a product is fastest, its reduction included.
 int dense_splits(int64_t m, int64_t n, int64_t k);
 // parts[y] = a[:, slice y] w[:, slice y]^T in fp32, (splits, m, n): k / splits wide slices.

@@ -1768,6 +1768,15 @@ extern "C" int kx_gemm_splits(int64_t m, int64_t n, int64_t k, int* splits) {
   return KX_OK;
 }
 
+extern "C" int kx_gemm_kernels(int64_t m, int64_t n, int64_t k, int* count) {
+  KX_REQUIRE(count, "kx_gemm_kernels: null result");
+  KX_REQUIRE(m >= 0 && n >= 0 && k > 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 30),
+             "kx_gemm_kernels: bad shape (%lld, %lld, %lld)", (long long)m, (long long)n, (long long)k);
+  if (m == 0 || n == 0) *count = 0;
+  else *count = m <= FEW_ROWS || (n <= 64 && k % 128 == 0) || k % DENSE_BK ? 1 : dense_kernels(m, n, k);
+  return KX_OK;
+}
+
 extern "C" int kx_gemm_splitk_noalloc_bf16(const void* a, int64_t lda, const void* w, int64_t ldw,
                                            const void* bias, void* c, int64_t ldc, int64_t m, int64_t n, int64_t k,
                                            int epilogue, const void* resid, int64_t ldr, const float* gate,

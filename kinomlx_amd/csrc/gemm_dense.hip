@@ -846,6 +846,12 @@ int dense_splits(int64_t m, int64_t n, int64_t k) {
   return best;
 }
 
+int dense_kernels(int64_t m, int64_t n, int64_t k) {
+  int count = 0;
+  run_rows(m, n, k, [&](int64_t, int64_t, int) { ++count; });
+  return count;
+}
+
 void launch_dense(bool half, const uint16_t* a, int64_t lda, const uint16_t* w, int64_t ldw, void* c, int64_t ldc,
                   int m, int n, int k, const Epilogue& epi, hipStream_t s) {
   run_rows(m, n, k, [&](int64_t row0, int64_t rows, int tile) {
