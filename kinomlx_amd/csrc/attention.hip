@@ -186,8 +186,10 @@ enum KeySplit { KEYS_ALL = 0, KEYS_SLICES = 1, KEYS_TAIL = 2 };
 // once and stays there while the workgroup runs up to qpw consecutive query tiles of its head; the
 // waves need no barrier after the copy, so one wave's query load and output store overlap the
 // other waves' products.
-template <bool H, int D, int BIAS, int SPLIT, bool RES = false>
-__global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
+//
+// NW = 8: query tiles of 256 for calls that fit one round with them (see small_tiles), two waves per SIMD.
+template <bool H, int D, int BIAS, int SPLIT, bool RES = false, int NW = NWAVE>
+__global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(
     const uint16_t* __restrict__ Q, int64_t ldq, const uint16_t* __restrict__ K, int64_t ldk,
     const uint16_t* __restrict__ V, int64_t ldv, uint16_t* __restrict__ O, int64_t ldo, int tq,
     int tk_all, int heads, int kv_group, float scale_log2, const uint16_t* __restrict__ gate,
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
   constexpr int STAGE = 2 * TILE;
   constexpr int INST = 2 * BKV / RPI;     // DMA instructions per stage (K then V)
   constexpr int PER = INST / NDMA;        // per DMA wave
-  static_assert(PER * NDMA == INST, "DMA split");
+  static_assert(PER * NDMA == INST && NW >= NDMA, "DMA split");
   const bool dma_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < NDMA;
   constexpr int QS = D / 16, DB = D / 32;
   constexpr bool PIPE = D == 128 && BIAS != BIAS_FULL;  // the software-pipelined key loop
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
       const int u = xcd_remap(blockIdx.x - split.full, gridDim.x - split.full);
       slice = u / split.tail;
       t = split.full + u % split.tail;
-      part_row = u * BQ;
+      part_row = u * (32 * NW);
     }
   } else {
     t = xcd_remap(blockIdx.x, gridDim.x);
@@ -243,7 +245,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
   const char* Kb = reinterpret_cast<const char*>(K + ((int64_t)b * tk_all + j_begin) * ldk + (int64_t)hk * D);
   const char* Vb = reinterpret_cast<const char*>(V + ((int64_t)b * tk_all + j_begin) * ldv + (int64_t)hk * D);
 
-  int q0 = qt * BQ + wave * 32;
+  int q0 = qt * (32 * NW) + wave * 32;
   int qrow = min(q0 + lrow, tq - 1);
   bf16x8 qf[QS];
 #pragma unroll
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
     auto buf = [&](int t) { return smem + (t % NSTAGE) * STAGE; };
     if constexpr (BIAS == BIAS_KEYS) {
       const uint16_t* brow = bias.ptr + (int64_t)b * bias.bs + (int64_t)h * bias.hs + j_begin;
-      for (int i = tid; i < ntiles * BKV; i += NWAVE * 64) {
+      for (int i = tid; i < ntiles * BKV; i += NW * 64) {
         const float add = i < tk ? e2f<H>(brow[i]) * bias.mul : 0.0f;
         key_bias[i] = add < -1e20f ? REMOVED : add;
       }
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_fwd_kernel(
       const int nq = min(qpw, qtiles - qt);
       for (int qi = 0; qi < nq; ++qi) {
         if (qi > 0) {
-          q0 += BQ;
+          q0 += (32 * NW);
           qrow = min(q0 + lrow, tq - 1);
 #pragma unroll
           for (int st = 0; st < QS; ++st)
@@ -722,12 +724,12 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
   *reinterpret_cast<uint2*>(O + ((int64_t)b * tq + q) * ldo + (int64_t)h * D + d) = w2;
 }
 
-template <bool H, int D, int BIAS, int SPLIT, bool RES = false>
+template <bool H, int D, int BIAS, int SPLIT, bool RES = false, int NW = NWAVE>
 void launch_attn_t(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, void* o,
                    int64_t ldo, int64_t tq, int64_t tk, int64_t heads, int64_t kv_heads, float scale,
                    const void* gate, int64_t ld_gate, ScoreBias bias, SplitOut split, dim3 grid, int qtiles,
                    hipStream_t s, int qpw = 1) {
-  attn_fwd_kernel<H, D, BIAS, SPLIT, RES><<<grid, NWAVE * 64, 0, s>>>(
+  attn_fwd_kernel<H, D, BIAS, SPLIT, RES, NW><<<grid, NW * 64, 0, s>>>(
       (const uint16_t*)q, ldq, (const uint16_t*)k, ldk, (const uint16_t*)v, ldv, (uint16_t*)o, ldo, (int)tq,
       (int)tk, (int)heads, (int)(heads / kv_heads), scale * 1.4426950408889634f, (const uint16_t*)gate, ld_gate,
       qtiles, qpw, bias, split);
@@ -749,6 +751,12 @@ int resident_qpw(int64_t qtiles, int64_t heads_total) {
   }
   return best;
 }
+
+// Whether the plain D = 128 form runs on 256-query tiles (8 waves): where they still fit one round of 256
+// workgroups, each workgroup then has less to do and more CUs have a workgroup. 32 heads, as many
+// keys as queries, 384 / 256-query tiles in us: 480 24.3 / 20.1, 1000 39.2 / 32.9, 1900 68.1 / 67.1; 24 heads of 2305
+// 82.2 / 75.6. Past one round they lose (2300 x 32 heads: 87 / 137), and 128-query tiles gain at most 1 us more.
+bool small_tiles(int64_t tq, int64_t heads_total) { return (tq + 255) / 256 * heads_total <= 256; }
 
 template <bool H, int D>
 int launch_attn(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
@@ -803,6 +811,12 @@ int launch_attn(const void* q, int64_t ldq, const void* k, int64_t ldk, const vo
     else launch(none, no, resident, rgrid, qpw);
   } else if (keys) {
     launch(by_key, no, stream, grid, 1);
+  } else if (D == 128 && small_tiles(tq, heads * batch)) {
+    constexpr int NW = D == 128 ? 8 : NWAVE;
+    const int tiles = (int)((tq + 32 * NW - 1) / (32 * NW));
+    launch_attn_t<H, D, BIAS_NONE, KEYS_ALL, false, NW>(q, ldq, k, ldk, v, ldv, o, ldo, tq, tk, heads, kv_heads, scale,
+                                                        gate, ld_gate, bias, split,
+                                                        dim3((unsigned)(tiles * heads * batch)), tiles, s);
   } else {
     launch(none, no, stream, grid, 1);
   }

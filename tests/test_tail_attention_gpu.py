@@ -58,6 +58,25 @@ def test_tail_slices(device, dtype, batch, heads, kv, tq, tk, splits):
         assert ((a.view(ref.shape) - ref).abs() <= 1.01 * tol).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("batch", "heads", "kv", "tq", "tk"), [
+    (1, 3, 3, 1, 257), (2, 4, 2, 256, 300), (1, 4, 4, 257, 1000), (1, 86, 86, 513, 321),  # within one round
+    (1, 86, 86, 640, 321)])                                                               # past it: 384-query tiles
+def test_small_query_tiles(device, dtype, batch, heads, kv, tq, tk):
+    """256-query tiles against the key-sliced form, which keeps 384-query tiles."""
+    q, k, v = (_t(device, (batch, n, h * 128), i, dtype) for i, (n, h) in enumerate(((tq, heads), (tk, kv), (tk, kv))))
+    gate = _t(device, (batch * tq, heads), 4, dtype)
+    got = _launch("kx_attention_gqa_fwd", q, k, v, heads, kv, gate)
+    work = torch.empty(2 * batch * heads * tq * 130, dtype=torch.float32, device=device)
+    sliced = _launch("kx_attention_split_fwd", q, k, v, heads, kv, gate, None, 0, 0, 0, work.data_ptr(),
+                     work.numel() * 4, 2)
+    # both round P to 16 bits (u) against their own running max, and the output once
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    size = v.float().abs().amax() * gate.float().abs().view(batch, tq, heads, 1)
+    diff = (got.float() - sliced.float()).abs().view(batch, tq, heads, 128)
+    assert (diff <= 6 * u * size).all()
+
+
 def test_rule_and_refusals(device):
     assert _lib.attention_tail(1, 4608, 4608, 32) == 2
     assert _lib.attention_tail(1, 9216, 9216, 32) == 1   # whole rounds
